@@ -244,9 +244,9 @@ static b1::LinearArgs linear_args(const float *act, int64_t lda, const void *w, 
     return a;
 }
 
-// The workspace the kernel linear_impl picks for these arguments can use:
-// the FAST GEMM's range-safe packing and split-K partials; none for the
-// small-M kernel and EXACT mode.
+// The workspace size the queries report for these arguments: the FAST
+// GEMM's range-safe packing and gemm_partial_bytes; none for the small-M
+// kernel and EXACT mode.
 static size_t linear_need(const b1::LinearArgs &a, int mode, int num_cus) {
     if (mode == BONSAI_B1_MODE_EXACT || mode == BONSAI_B1_MODE_GEMV) return 0;
     if (mode != BONSAI_B1_MODE_GEMM && b1::gemv_supported(a)) return 0;
@@ -277,7 +277,7 @@ static int linear_impl(const float *act, int64_t lda, const void *w, int in_dim,
         }
     };
     auto gemm = [&]() {
-        workspace(linear_need(a, mode, dev->num_cus));
+        workspace(b1::gemm_workspace_bytes(a));
         return b1::launch_gemm(a, dev->num_cus, ws, ws_bytes, stream);
     };
     auto gemv = [&]() { return b1::launch_gemv(a, dev->num_cus, stream); };
@@ -327,8 +327,7 @@ size_t bonsai_b1_workspace_bytes(int batch, int in_dim, int out_dim, int mode) {
     a.w = reinterpret_cast<const uint8_t *>(uintptr_t(256));
     // the small-M kernel converts the activations itself
     if (mode == BONSAI_B1_MODE_GEMV || (mode != BONSAI_B1_MODE_GEMM && batch <= b1::kGemvMaxM)) return 0;
-    // the range-safe packing, then (on a device where the shape splits
-    // along K) the split-K partials
+    // the range-safe packing, then gemm_partial_bytes (0 without a device)
     const DeviceInfo *dev = current_device(nullptr);
     return b1::gemm_workspace_bytes_total(a, dev ? dev->num_cus : 0);
 }
@@ -491,16 +490,13 @@ size_t bonsai_b1_linear_packed_workspace_bytes(int batch, int in_dim, int out_di
     if (batch <= 0 || in_dim <= 0 || out_dim <= 0 || !b1::gemm_packed_ok(batch, in_dim, out_dim)) return 0;
     if (b1::gemv_packed_ok(batch, in_dim, out_dim)) return 0;
     const DeviceInfo *dev = current_device(nullptr);
-    const int splits = dev ? b1::gemm_splits(batch, in_dim, out_dim, dev->num_cus) : 1;
-    return b1::gemm_split_bytes(batch, out_dim, splits);
+    return b1::gemm_partial_bytes(batch, in_dim, out_dim, out_dim, dev ? dev->num_cus : 0);
 }
 
-// Shared body of the packed entry points.  ws_mode: 0 = library-owned
-// workspace for the split-K partials, 1 = caller's (may be NULL / small:
-// then unsplit).
+// Shared body of the packed entry points (ws: checked, not used).
 static int linear_packed_impl(const void *packed_act, const float *rsc, const void *w, int in_dim, int out_dim,
-                              int batch, float *out, int64_t ldo, int32_t *nonfinite, int ws_mode, void *ws,
-                              size_t ws_bytes, hipStream_t stream) {
+                              int batch, float *out, int64_t ldo, int32_t *nonfinite, const void *ws,
+                              hipStream_t stream) {
     if (in_dim <= 0 || out_dim <= 0 || batch < 0 || ldo < out_dim) return BONSAI_B1_ERR_ARG;
     if (batch > 0 && (!packed_act || !w || !out)) return BONSAI_B1_ERR_ARG;
     if ((reinterpret_cast<uintptr_t>(packed_act) & 15u) || (reinterpret_cast<uintptr_t>(w) & 3u) ||
@@ -518,24 +514,10 @@ static int linear_packed_impl(const void *packed_act, const float *rsc, const vo
         e = b1::launch_gemv_packed(packed_act, wb, in_dim, out_dim, batch, out, ldo, nonfinite, dev->num_cus, stream,
                                    rsc);
     } else {
-        // split along K as bonsai_b1_linear_f32 splits the same shape, when
-        // the partials have room: the two entries then agree bit for bit
-        const int splits = b1::gemm_splits(batch, in_dim, out_dim, dev->num_cus);
-        const size_t need = b1::gemm_split_bytes(batch, out_dim, splits);
-        WsLease lease;
-        if (need > 0 && ws_mode == 0) {
-            lease.acquire(dev, stream, need);
-            ws = lease.ptr();
-            ws_bytes = ws ? need : 0;
-        }
         b1::GemmEpi epi;
         epi.rsc = rsc;
-        if (need > 0 && ws && ws_bytes >= need)
-            e = b1::launch_gemm_packed_split(packed_act, wb, in_dim, out_dim, batch, out, ldo, nonfinite,
-                                             dev->num_cus, splits, ws, stream, rsc);
-        else
-            e = b1::launch_gemm_packed_epi(packed_act, wb, in_dim, out_dim, batch, out, ldo, nonfinite, dev->num_cus,
-                                           0, epi, stream);
+        e = b1::launch_gemm_packed_epi(packed_act, wb, in_dim, out_dim, batch, out, ldo, nonfinite, dev->num_cus,
+                                       b1::gemm_kranges(batch, in_dim, out_dim, dev->num_cus), 0, epi, stream);
     }
     return e == hipSuccess ? BONSAI_B1_OK : BONSAI_B1_ERR_HIP;
 }
@@ -544,21 +526,19 @@ int bonsai_b1_linear_packed_f16_scaled(const void *packed_act, const float *row_
                                        int out_dim, int batch, float *out, int64_t ldo, int32_t *nonfinite,
                                        hipStream_t stream) {
     if (batch > 0 && !row_scale) return BONSAI_B1_ERR_ARG;
-    return linear_packed_impl(packed_act, row_scale, w, in_dim, out_dim, batch, out, ldo, nonfinite, 0, nullptr, 0,
-                              stream);
+    return linear_packed_impl(packed_act, row_scale, w, in_dim, out_dim, batch, out, ldo, nonfinite, nullptr, stream);
 }
 
 int bonsai_b1_linear_packed_f16(const void *packed_act, const void *w, int in_dim, int out_dim, int batch,
                                 float *out, int64_t ldo, int32_t *nonfinite, hipStream_t stream) {
-    return linear_packed_impl(packed_act, nullptr, w, in_dim, out_dim, batch, out, ldo, nonfinite, 0, nullptr, 0,
-                              stream);
+    return linear_packed_impl(packed_act, nullptr, w, in_dim, out_dim, batch, out, ldo, nonfinite, nullptr, stream);
 }
 
 int bonsai_b1_linear_packed_f16_ws(const void *packed_act, const void *w, int in_dim, int out_dim, int batch,
                                    float *out, int64_t ldo, int32_t *nonfinite, void *workspace,
                                    size_t workspace_bytes, hipStream_t stream) {
-    return linear_packed_impl(packed_act, nullptr, w, in_dim, out_dim, batch, out, ldo, nonfinite, 1, workspace,
-                              workspace_bytes, stream);
+    (void)workspace_bytes;
+    return linear_packed_impl(packed_act, nullptr, w, in_dim, out_dim, batch, out, ldo, nonfinite, workspace, stream);
 }
 
 // Checks an epilogue against a linear of out_dim outputs (weight rows) and
@@ -654,7 +634,8 @@ int bonsai_b1_linear_packed_f16_epi(const void *packed_act, const void *w, int i
     if (!dev) return BONSAI_B1_ERR_DEVICE;
     if (batch == 0) return BONSAI_B1_OK;
     return b1::launch_gemm_packed_epi(packed_act, static_cast<const uint8_t *>(w), in_dim, out_dim, batch, out, ldo,
-                                      nonfinite, dev->num_cus, kind, g, stream) == hipSuccess
+                                      nonfinite, dev->num_cus,
+                                      b1::gemm_kranges(batch, in_dim, out_dim, dev->num_cus), kind, g, stream) == hipSuccess
                ? BONSAI_B1_OK
                : BONSAI_B1_ERR_HIP;
 }
@@ -694,7 +675,8 @@ int bonsai_b1_linear_packed_f16_to_packed(const void *packed_act, const void *w,
     if (!dev) return BONSAI_B1_ERR_DEVICE;
     if (batch == 0) return BONSAI_B1_OK;
     return b1::launch_gemm_packed_epi(packed_act, static_cast<const uint8_t *>(w), in_dim, out_dim, batch, out, ldo,
-                                      nonfinite, dev->num_cus, kind, g, stream) == hipSuccess
+                                      nonfinite, dev->num_cus,
+                                      b1::gemm_kranges(batch, in_dim, out_dim, dev->num_cus), kind, g, stream) == hipSuccess
                ? BONSAI_B1_OK
                : BONSAI_B1_ERR_HIP;
 }
@@ -771,7 +753,7 @@ int bonsai_b1_linear_epi_f32(const float *act, int64_t lda, const void *w, int i
         g.rsc = b1::pack_area_rsc(workspace, batch, in_dim);
         if (e == hipSuccess)
             e = b1::launch_gemm_packed_epi(workspace, a.w, in_dim, out_dim, batch, out, ldo, nonfinite, dev->num_cus,
-                                           kind, g, stream);
+                                           b1::gemm_kranges(batch, in_dim, out_dim, dev->num_cus), kind, g, stream);
     } else {
         // the linear into the workspace (a kernel that needs no workspace of
         // its own), then the epilogue pass
@@ -852,14 +834,14 @@ static size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 // The ops from i on that run as one GEMM with op i, on the packed path:
 // consecutive plain ops on the same input whose weights follow each other in
 // memory and whose outputs are adjacent column ranges of one row stride (q/k/v
-// with concatenated weights, src/diffuser_graph.cpp:354-361), split along K
-// as op i alone would be, unless an output overlaps the input they all read.
+// with concatenated weights, src/diffuser_graph.cpp:354-361), in the K ranges
+// each would run with alone, unless an output overlaps the input they all read.
 // Returns the last op of the run; *n_sum is its output width.
 template <class OpAt>
 static int fuse_span(int n_ops, int mode, int num_cus, OpAt at, int i, int *n_sum) {
     const BatchOp bi = at(i);
     const b1::LinearArgs a = batch_args(*bi.op);
-    const int splits = b1::gemm_splits(a.M, a.K, a.N, num_cus);
+    const int kranges = b1::gemm_kranges(a.M, a.K, a.N, num_cus);
     int last = i;
     *n_sum = a.N;
     while (epi_kind(bi.epi) == BONSAI_B1_EPI_NONE && last + 1 < n_ops) {
@@ -875,13 +857,7 @@ static int fuse_span(int n_ops, int mode, int num_cus, OpAt at, int i, int *n_su
             !b1::gemm_packed_ok(a.M, a.K, *n_sum + q.w->out_dim))
             break;
         const b1::LinearArgs qa = batch_args(q);
-        if (batch_path(qa, mode) != BatchPath::Packed || b1::gemm_splits(qa.M, qa.K, qa.N, num_cus) != splits) break;
-        // the concatenated GEMM runs the tile kernel each part would (the
-        // two sum K in different orders)
-        const int tk = b1::gemm_tiles(a.M, a.K, a.N, num_cus);
-        if (b1::gemm_tiles(qa.M, qa.K, qa.N, num_cus) != tk ||
-            b1::gemm_tiles(a.M, a.K, *n_sum + q.w->out_dim, num_cus) != tk)
-            break;
+        if (batch_path(qa, mode) != BatchPath::Packed || b1::gemm_kranges(qa.M, qa.K, qa.N, num_cus) != kranges) break;
         *n_sum += q.w->out_dim;
         ++last;
     }
@@ -952,9 +928,10 @@ static int gemv_span(int n_ops, int mode, OpAt at, int i, b1::GemvGroupOp *ops, 
 
 // Workspace areas of a batch, laid out [pack][split][y], each 256-byte
 // aligned: the largest range-safe packing among its packed GEMMs and
-// grouped small-M runs of more than kGemvGroupF32MaxM tokens, the largest split-K partial area among its plain packed GEMMs
-// (fused runs included), and the largest fp32 linear output among its ops
-// whose epilogue runs as a separate pass (the other paths).
+// grouped small-M runs of more than kGemvGroupF32MaxM tokens, the largest
+// gemm_partial_bytes among its plain packed GEMMs (fused runs included; part
+// of the reported size only), and the largest fp32 linear output among its
+// ops whose epilogue runs as a separate pass (the other paths).
 struct BatchAreas {
     size_t pack = 0, split = 0, y = 0;
     size_t split_off() const { return round256(pack); }
@@ -984,8 +961,7 @@ static BatchAreas batch_areas(int n_ops, int mode, int num_cus, OpAt at, bool pa
             if (epi_kind(b.epi) == BONSAI_B1_EPI_NONE) {
                 int n_sum;
                 const int last = fuse_span(n_ops, mode, num_cus, at, i, &n_sum);
-                r.split = std::max(r.split,
-                                   b1::gemm_split_bytes(a.M, n_sum, b1::gemm_splits(a.M, a.K, a.N, num_cus)));
+                r.split = std::max(r.split, b1::gemm_partial_bytes(a.M, a.K, a.N, n_sum, num_cus));
                 i = last;
             }
         } else if (epi_kind(b.epi) != BONSAI_B1_EPI_NONE) {
@@ -1024,7 +1000,8 @@ static int batch_run(int n_ops, int mode, int32_t *nonfinite, void *workspace, s
     bool pack_groups = true;
     if (areas.need() > 0) {
         if (!workspace) {
-            lease.acquire(dev, stream, areas.need());
+            areas.split = 0; // no kernel uses that area
+            if (areas.need() > 0) lease.acquire(dev, stream, areas.need());
             workspace = lease.ptr();
             workspace_bytes = workspace ? areas.need() : 0;
             if (!workspace) {
@@ -1040,8 +1017,7 @@ static int batch_run(int n_ops, int mode, int32_t *nonfinite, void *workspace, s
         }
     }
     if (areas.need() > 0) {
-        // a workspace without room for the split-K partials runs every GEMM
-        // unsplit (the same outputs up to the order of the K summation)
+        // (a workspace need not hold that area)
         if (workspace && workspace_bytes < areas.need()) areas.split = 0;
         if (!workspace || workspace_bytes < areas.need() || (reinterpret_cast<uintptr_t>(workspace) & 15u))
             return BONSAI_B1_ERR_ARG;
@@ -1081,7 +1057,6 @@ static int batch_run(int n_ops, int mode, int32_t *nonfinite, void *workspace, s
         }
     }
     float *ybuf = areas.y ? reinterpret_cast<float *>(static_cast<uint8_t *>(workspace) + areas.y_off()) : nullptr;
-    void *split_area = areas.split ? static_cast<uint8_t *>(workspace) + areas.split_off() : nullptr;
     // The packed activations in the workspace belong to (act, lda, batch, K).
     const float *packed_act = nullptr;
     int64_t packed_lda = 0;
@@ -1144,16 +1119,10 @@ static int batch_run(int n_ops, int mode, int32_t *nonfinite, void *workspace, s
         } else {
             int n_sum;
             const int last = fuse_span(n_ops, mode, dev->num_cus, at, i, &n_sum);
-            const int splits = kind == BONSAI_B1_EPI_NONE ? b1::gemm_splits(a.M, a.K, a.N, dev->num_cus) : 1;
             g.rsc = rsc;
-            if (e == hipSuccess) {
-                if (splits > 1 && split_area && areas.split >= b1::gemm_split_bytes(a.M, n_sum, splits))
-                    e = b1::launch_gemm_packed_split(workspace, a.w, a.K, n_sum, a.M, a.out, a.ldo, nonfinite,
-                                                     dev->num_cus, splits, split_area, stream, rsc);
-                else
-                    e = b1::launch_gemm_packed_epi(workspace, a.w, a.K, n_sum, a.M, a.out, a.ldo, nonfinite,
-                                                   dev->num_cus, kind, g, stream);
-            }
+            if (e == hipSuccess)
+                e = b1::launch_gemm_packed_epi(workspace, a.w, a.K, n_sum, a.M, a.out, a.ldo, nonfinite, dev->num_cus,
+                                               b1::gemm_kranges(a.M, a.K, a.N, dev->num_cus), kind, g, stream);
             if (last > i) out_cols = n_sum;
             i = last;
         }

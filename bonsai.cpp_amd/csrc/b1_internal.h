@@ -50,29 +50,30 @@ hipError_t launch_exact(const LinearArgs &a, int num_cus, hipStream_t s);
 // staging each tile, and launch_fixup_rows follows.
 bool gemm_supported(const LinearArgs &a);
 size_t gemm_workspace_bytes(const LinearArgs &a);
-// With room for the split-K partials after the packing (256-byte aligned),
-// launch_gemm splits K when gemm_splits says so.
+// The size callers are told: the packing and the area gemm_partial_bytes
+// describes (which no kernel uses).
 size_t gemm_workspace_bytes_total(const LinearArgs &a, int num_cus);
 hipError_t launch_gemm(const LinearArgs &a, int num_cus, void *workspace, size_t ws_bytes, hipStream_t s);
 
-// Split-K for plain GEMMs whose tiles would leave most CUs idle: the number
-// of K ranges (1 = none; a function of the shape and CU count only, so
-// every caller splits a given shape the same way) and the fp32 partial
-// area it needs (splits x M x N rounded up to 4 columns).
-int gemm_splits(int M, int K, int N, int num_cus);
-size_t gemm_split_bytes(int M, int N, int splits);
-// The tile kernel of the packed GEMM with the plain, gate-residual or
-// packed-output (GELU or none) epilogue: 0 b1_gemm_kernel, 128 x 512 tiles
-// (any shape; 64-row tiles for a short last round, split-K for few tiles);
-// 1 b1_gemm16_kernel 144 x 384 and 2 b1_gemm16_kernel 128 x 384 (16x16x32
-// MFMAs; full tiles, K % 384 == 0, no split), whichever needs the fewest
-// rounds on num_cus CUs, counting a BM x BN tile as BM BN / 65536 of a
-// 128 x 512 round; ties stay on 0.  A function of the shape and CU count
-// only, so every entry point picks alike, for every epilogue (the packed
-// output's SwiGLU columns need split % 384 == 0 for the 16x16 kernels;
-// otherwise kernel 0).  The kernels sum K in different orders (the same to
-// ~1e-6 relative).
-int gemm_tiles(int M, int K, int N, int num_cus);
+// Bytes the size queries report beyond the packing (n_sum: the width of a
+// run of linears issued as one).
+size_t gemm_partial_bytes(int M, int K, int N, int n_sum, int num_cus);
+
+// The number of contiguous K ranges a packed GEMM sums separately and then
+// adds in order (1, 2, 4 or 8), a function of the shape and CU count only,
+// so that every entry point and epilogue gives a linear the same bits: 1
+// when 64 x 192 tiles give at least 1.25 work-groups a CU, else as many as
+// fill the CUs with 64-row tiles of 48 (8 ranges), 96 (4) or 192 (2)
+// columns, and no range shorter than 384.  With one range every kernel of
+// the packed GEMM gives the same bits (the 16x16x32 and 32x32x16 MFMAs add
+// a K-slot order's products alike), so which of them runs is free.
+int gemm_kranges(int M, int K, int N, int num_cus);
+// The K-range tile GEMM (b1_tile_gemm.h), any K % 128 == 0 (K % 64 == 0 for
+// 2, 4 and 8 ranges), and its modelled time for one range in us.
+hipError_t launch_tile_gemm(const void *packed, const uint8_t *w, int K, int N, int M, float *out, int64_t ldo,
+                            int32_t *nonfinite, int num_cus, int kranges, int kind, const GemmEpi &epi,
+                            hipStream_t s);
+double tile_gemm_us(int M, int K, int N, int num_cus);
 
 // The two halves of the workspace path.  Packed activations: u32 word
 // (row m, 16 j + d) = fp16(a[m][32 j + d]) | fp16(a[m][32 j + d + 16]) << 16,
@@ -83,14 +84,6 @@ int gemm_tiles(int M, int K, int N, int num_cus);
 bool pack_supported(const float *act, int64_t lda, int M, int K);
 hipError_t launch_pack(const float *act, int64_t lda, int M, int K, void *packed, int64_t ldp, hipStream_t s);
 bool gemm_packed_ok(int M, int K, int N);
-hipError_t launch_gemm_packed(const void *packed, const uint8_t *w, int K, int N, int M, float *out, int64_t ldo,
-                              int32_t *nonfinite, int num_cus, hipStream_t s);
-// The same split into `splits` K ranges (a divisor of K / 384) with the
-// partials in `partials` (gemm_split_bytes, 16-byte aligned), summed in
-// order by a second kernel.
-hipError_t launch_gemm_packed_split(const void *packed, const uint8_t *w, int K, int N, int M, float *out,
-                                    int64_t ldo, int32_t *nonfinite, int num_cus, int splits, void *partials,
-                                    hipStream_t s, const float *rsc = nullptr);
 
 // Range-safe packing of the fp32 entry points' activations into a packing
 // area of pack_area_bytes(M, K) bytes (16-byte aligned): the packed fp16
@@ -116,8 +109,8 @@ hipError_t launch_fixup_rows(const LinearArgs &a, hipStream_t s);
 // 3 fp32 / packed fp16 columns with N % 32 == 0; with split > 0, out 16-byte
 // aligned and ldo % 4 == 0).
 hipError_t launch_gemm_packed_epi(const void *packed, const uint8_t *w, int K, int N, int M, float *out,
-                                  int64_t ldo, int32_t *nonfinite, int num_cus, int kind, const GemmEpi &epi,
-                                  hipStream_t s);
+                                  int64_t ldo, int32_t *nonfinite, int num_cus, int kranges, int kind,
+                                  const GemmEpi &epi, hipStream_t s);
 
 // The epilogue (kind 1 or 2) as a separate pass over y [M][ldy] (N columns
 // of y; kind 2 writes glu_h of them).

@@ -34,202 +34,11 @@
 
 #include <mutex>
 
+#include "b1_device.h"
 #include "b1_internal.h"
 
 namespace b1 {
 namespace {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-typedef float float2v __attribute__((ext_vector_type(2)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-constexpr uint32_t kSignPair = 0x80008000u;
-
-// Bits of m: ~(x ^ y); other bits: y.  One v_bitop3_b32, whose 8-bit table
-// is indexed by (x_bit << 2) | (m_bit << 1) | y_bit: 0xa6 = {0,1,1,0,0,1,0,1}
-// for indices 0..7.  Through the compiler builtin, not inline asm: the
-// compiler must see the VALU write, or it cannot insert the wait states an
-// MFMA reading the result as a source operand needs (an MFMA issued too
-// soon after an asm-hidden write read stale operands here).
-__device__ __forceinline__ uint32_t xnor_sel(uint32_t m, uint32_t x, uint32_t y) {
-    return __builtin_amdgcn_bitop3_b32(x, m, y, 0xa6);
-}
-
-// (lo, hi) -> packed fp16 pair, round to nearest even (v_cvt_pk_f16_f32).
-__device__ __forceinline__ uint32_t pack_f16(float lo, float hi) {
-    float2v v = {lo, hi};
-    half2v h = __builtin_convertvector(v, half2v);
-    return __builtin_bit_cast(uint32_t, h);
-}
-
-// fp32 -> fp16 bits of one value, rounded once from the fp32 value: the
-// empty asm keeps the compiler from folding the multiply that produced x
-// into the conversion (v_fma_mixlo_f16 rounds the exact product to fp16
-// once, which differs from the producer passes' fp32-then-fp16 rounding in
-// the rare products an fp32 rounding puts on an fp16 midpoint).
-__device__ __forceinline__ uint16_t half_bits(float x) {
-    asm("" : "+v"(x));
-    return (uint16_t)pack_f16(x, 0.0f);
-}
-
-// (lo, hi) -> packed fp16 pair, each rounded once from its fp32 value (the
-// fold half_bits keeps out, for two values).
-__device__ __forceinline__ uint32_t pack_f16_rounded(float lo, float hi) {
-    asm("" : "+v"(lo), "+v"(hi));
-    return pack_f16(lo, hi);
-}
-
-// max(m, |a|, |b|) in one v_max3_f32: the running largest magnitude of the
-// activations a lane converts, against fp16's range (a quiet NaN operand is
-// passed over, as IEEE maxNum does: a NaN does not count as out of range).
-__device__ __forceinline__ float absmax3(float m, float a, float b) {
-    float r;
-    asm("v_max3_f32 %0, %1, |%2|, |%3|" : "=v"(r) : "v"(m), "v"(a), "v"(b));
-    return r;
-}
-// fp32 magnitudes from this on round to fp16 infinity
-constexpr float kF16Overflow = 65520.0f;
-
-// s_waitcnt vmcnt(N) leaving expcnt and lgkmcnt alone (gfx9 encoding:
-// vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt range");
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-
-// Waits for this wave's LDS operations only (vmcnt and expcnt left open).
-__device__ __forceinline__ void wait_lgkmcnt0() {
-    __builtin_amdgcn_s_waitcnt(0xF | (0x3 << 14) | (0x7 << 4) | (0x0 << 8));
-}
-
-// Work-group barrier that does not drain outstanding global->LDS loads
-// (__syncthreads() would add s_waitcnt vmcnt(0) while LDS-DMA is pending).
-// Each wave waits for its own loads with wait_vmcnt<> before arriving.
-__device__ __forceinline__ void lds_barrier() {
-    asm volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-}
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-
-// Global -> LDS copies without VGPR staging.  `lds` must be wave-uniform
-// (it goes through M0).  Lane i's 16 bytes land at lds + 16 i; 12-byte
-// loads also land at lds + 16 i (a 16-byte lane stride, measured on gfx950
-// for the global and the buffer forms), leaving 4 bytes untouched per lane.
-// Kept as plain device functions: a kernel template that calls these
-// builtins directly loses its host-side launch stub.
-// global_load_lds_dword: lane i's 4 bytes land at lds + 4 i.  The compiler
-// treats this global form as a FLAT access that may touch LDS, and with one
-// in a kernel it makes every LDS wait of that kernel a full lgkmcnt(0).  In
-// the GEMM (its row-scale copy) the buffer form instead gives waits that
-// count only the reads a step needs, and it measured no faster (252.9-253.4
-// vs 253.1 us at M=4096 K=3072 N=12288, 0.3-0.6 % slower on four other
-// shapes, bit-identical): the fragment reads' latency is already covered.
-__device__ __forceinline__ void dma_lds4(const void *src, void *lds) {
-    __builtin_amdgcn_global_load_lds(src, (lds_void_t *)lds, 4, 0, 0);
-}
-
-// Raw buffer loads with range checking (offsets at or past num_records read
-// zeros); word 3 of the resource for gfx9-family raw buffers.
-constexpr int kBufferFlags = 0x00020000;
-// Cache policy of the GEMM's full-tile output stores: the default.  Each
-// 16-byte store covers 32 rows x 32 bytes, a quarter of each 128-byte line,
-// and L2 merges the four quarters before the line goes to memory; the
-// non-temporal policy sends each quarter on its own (355 vs ~267 us at
-// M=4096 K=3072 N=12288).
-#ifndef B1_STORE_AUX
-#define B1_STORE_AUX 0
-#endif
-constexpr int kStoreNT = B1_STORE_AUX;
-// A 16-byte buffer store followed by 5 wait states before any instruction
-// may rewrite its data registers.  A store of more than 8 bytes reads its
-// data in the cycles after it issues; the compiler inserts that gap only
-// for stores whose soffset is not a register, and the epilogue stores carry
-// their row offset in an SGPR.  Without it, a VALU write issued right after
-// such a store changed the stored values of some lanes (the SwiGLU
-// epilogue: 2272 of 786,432 outputs, different on every launch).  The asm
-// takes the data as an input, so its registers stay live until the nops
-// have issued, and its memory clobber keeps it after the store.
-template <int AUX>
-__device__ __forceinline__ void store16_guarded(u32x4 v, __amdgpu_buffer_rsrc_t rsrc, int voff, int soff) {
-    __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, voff, soff, AUX);
-    asm volatile("s_nop 4" ::"v"(v) : "memory");
-}
-
-// 16 bytes per lane from the buffer at byte offset voff, landing at
-// lds + 16 * lane (wave-uniform lds, through M0).
-__device__ __forceinline__ void dma_buf_lds16(__amdgpu_buffer_rsrc_t rsrc, void *lds, uint32_t voff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t *)lds, 16, voff, 0, 0, 0);
-}
-// The same, 16 or 12 bytes per lane (12-byte lanes also land 16 bytes
-// apart), with a wave-uniform byte offset soff (an SGPR) added to voff.  A
-// constant offset goes into soff, not the instruction's offset field: for
-// these loads the instruction offset moves the LDS destination as well.
-__device__ __forceinline__ void dma_buf_lds16s(__amdgpu_buffer_rsrc_t rsrc, void *lds, uint32_t voff, uint32_t soff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t *)lds, 16, voff, soff, 0, 0);
-}
-__device__ __forceinline__ void dma_buf_lds12s(__amdgpu_buffer_rsrc_t rsrc, void *lds, uint32_t voff, uint32_t soff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t *)lds, 12, voff, soff, 0, 0);
-}
-// 4 bytes per lane, landing at lds + 4 * lane.
-__device__ __forceinline__ void dma_buf_lds4(__amdgpu_buffer_rsrc_t rsrc, void *lds, uint32_t voff) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void_t *)lds, 4, voff, 0, 0, 0);
-}
-
-__device__ __forceinline__ uint32_t dup_lo16(uint32_t d) {
-    return __builtin_amdgcn_perm(d, d, 0x01000100u);
-}
-__device__ __forceinline__ uint32_t dup_hi16(uint32_t d) {
-    return __builtin_amdgcn_perm(d, d, 0x03020302u);
-}
-
-// Weight dword for fp16 pair slot (bits p and p+16 of `w`, p = 15 - sh):
-// each half is the fp16 scale with its sign flipped where the bit is 0.
-__device__ __forceinline__ uint32_t wpair(uint32_t w, int sh, uint32_t scale2) {
-    return xnor_sel(kSignPair, w << sh, scale2);
-}
-
-// One v_lshlrev_b64 of the pair (w, w >> 8): its low dword is w << SH and
-// its high dword carries bits d + 8 and d + 24 of w at 15 and 31 (d = 15 -
-// SH < 8), so that one shift serves the weight dwords of pairs d and d + 8.
-// A 64-bit shift costs what a 32-bit one does on gfx950 (measured: both
-// about 2 ns per wave instruction per SIMD with the SIMDs saturated, a
-// v_bitop3 1.2 ns); the compiler splits a constant 64-bit shift into two
-// 32-bit ops, hence the asm.  Its result only feeds VALU bit ops (no MFMA
-// operand hazard).
-template <int SH>
-__device__ __forceinline__ uint64_t shl64(uint64_t v) {
-    static_assert(SH >= 8 && SH <= 15, "pairs d < 8");
-    uint64_t r;
-    asm("v_lshlrev_b64 %0, %1, %2" : "=v"(r) : "I"(SH), "v"(v));
-    return r;
-}
-// The weight dwords of pairs 4T + j (lo) and 4T + j + 8 (hi), j = 0..3,
-// T = 0 or 1, from the sign word w and w8 = w >> 8: the same values as
-// wpair(w, 15 - 4T - j, scale2) and wpair(w, 7 - 4T - j, scale2).
-template <int T>
-__device__ __forceinline__ void wpair_quads(uint32_t w, uint32_t w8, uint32_t scale2, u32x4 &lo, u32x4 &hi) {
-    const uint64_t v = (uint64_t)w8 << 32 | w;
-    const uint64_t v0 = shl64<15 - 4 * T>(v), v1 = shl64<14 - 4 * T>(v), v2 = shl64<13 - 4 * T>(v),
-                   v3 = shl64<12 - 4 * T>(v);
-    lo[0] = xnor_sel(kSignPair, (uint32_t)v0, scale2);
-    lo[1] = xnor_sel(kSignPair, (uint32_t)v1, scale2);
-    lo[2] = xnor_sel(kSignPair, (uint32_t)v2, scale2);
-    lo[3] = xnor_sel(kSignPair, (uint32_t)v3, scale2);
-    hi[0] = xnor_sel(kSignPair, (uint32_t)(v0 >> 32), scale2);
-    hi[1] = xnor_sel(kSignPair, (uint32_t)(v1 >> 32), scale2);
-    hi[2] = xnor_sel(kSignPair, (uint32_t)(v2 >> 32), scale2);
-    hi[3] = xnor_sel(kSignPair, (uint32_t)(v3 >> 32), scale2);
-}
-
-__device__ __forceinline__ void count_nonfinite(int32_t *ctr, int bad) {
-    if (bad && ctr) atomicAdd(ctr, bad);
-}
 
 // ---------------------------------------------------------------- exact --
 
@@ -324,15 +133,6 @@ struct GemmCfg {
     static_assert(UNITS % NT == 0, "staging units must divide evenly");
     static_assert(WM % 32 == 0 && WN % 32 == 0, "32x32 sub-tiles");
 };
-
-// Work-groups are dispatched round-robin over the 8 XCDs (bid % 8).  Give
-// each XCD a contiguous run of tiles (N-fastest) so the work-groups resident
-// on one XCD share activation rows in that XCD's L2.
-__device__ __forceinline__ int xcd_tile(int bid, int nblk) {
-    const int xcd = bid & 7, loc = bid >> 3;
-    const int q = nblk >> 3, r = nblk & 7;
-    return xcd * q + min(xcd, r) + loc;
-}
 
 template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kernel(LinearArgs p, int tiles_n) {
@@ -515,20 +315,6 @@ __device__ __forceinline__ void store_f4(float *p, const floatx4 &v) {
 // two B1_0 linears costs one read and one half-size write (or, in the
 // GEMM's epilogue, nothing beyond the GEMM's own half-size output).
 //
-// Evaluated as x / (1 + e^(-2u)), the same function (1 + tanh(u) =
-// 2 / (1 + e^(-2u))), with e^(-2u) = 2^(x (c1 + c2 x^2)), c1 = -2
-// sqrt(2/pi) / ln 2 and c2 = 0.044715 c1: one hardware exp2 and one
-// reciprocal instead of a library tanh, which matters in the GEMM epilogue
-// where no MFMA work overlaps it.  Within 3e-7 max(1, |x|) of the float64
-// function (1-ulp exp2 and reciprocal included).  Large negative x: the
-// exponential overflows to inf and the result is -0; NaN stays NaN.
-__device__ __forceinline__ float gelu_tanh(float x) {
-    const float c1 = -2.30220819f;  // -2 sqrt(2/pi) log2(e)
-    const float c2 = -0.102943242f; // 0.044715 c1
-    const float t = x * __builtin_fmaf(c2, x * x, c1);
-    return x * __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(t));
-}
-
 // Four float4 units in flight per thread (loads first), non-temporal past
 // 128 MB: a grid of at most 8192 blocks walking one unit at a time ran
 // 81.2 us at 4608 x 12288 (2.8 TB/s read), this form 72.0 us.  In place
@@ -586,25 +372,6 @@ __global__ __launch_bounds__(256) void b1_gelu_pack_kernel(const float *__restri
         for (int j = 0; j < 4; ++j) v[j] = pack_f16(gelu_tanh(lo[j]), gelu_tanh(hi[j]));
         *reinterpret_cast<u32x4 *>(ah + (size_t)row * ldw + blk * 16 + c * 4) = v;
     }
-}
-
-// silu(x) = x / (1 + e^-x), in fp32 with the device library's expf.
-__device__ __forceinline__ float silu_f32(float x) {
-#pragma clang fp contract(off)
-    return x / (1.0f + expf(-x));
-}
-
-// r + g y as the reference's two ggml ops (a multiply, then an add), each
-// rounded to fp32: never contracted into one FMA.
-__device__ __forceinline__ float gate_residual(float r, float g, float y) {
-#pragma clang fp contract(off)
-    const float t = g * y;
-    return r + t;
-}
-
-__device__ __forceinline__ float mul_f32(float a, float b) {
-#pragma clang fp contract(off)
-    return a * b;
 }
 
 // SwiGLU (ggml_swiglu: silu of the first half of a row times its second
@@ -1086,8 +853,7 @@ __global__ __launch_bounds__((BN / WN) * 64, (BN / WN) >= 8 ? 2 : 1) void b1_gem
                                                                     const uint8_t *__restrict__ w, int K, int N,
                                                                     int M, float *__restrict__ out, int64_t ldo,
                                                                     int32_t *nonfinite, int tiles_m, int tiles_n,
-                                                                    int vec_store, GemmEpi epi, int ksplit,
-                                                                    int64_t pstride) {
+                                                                    int vec_store, GemmEpi epi) {
     using C = GemmLdsCfg<BM, BN, WN, STAGES>;
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
 
@@ -1095,13 +861,8 @@ __global__ __launch_bounds__((BN / WN) * 64, (BN / WN) >= 8 ? 2 : 1) void b1_gem
     // through M0 and must not depend on the lane.
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int li = lane & 31, g = lane >> 5;
-    // Work unit u: K range `split` = u / (tiles_m tiles_n) of ksplit equal
-    // ranges, output tile u % (tiles_m tiles_n).  With ksplit > 1 a unit's
-    // plain product goes to partial slice `split` (out + split * pstride),
-    // which a separate pass sums.
-    const int nstage = K / C::KC / ksplit; // stages per unit, a multiple of STAGES
+    const int nstage = K / C::KC; // a multiple of STAGES
     const int ntiles = tiles_m * tiles_n;
-    const int nunits = ntiles * ksplit;
     const uint32_t rs = (uint32_t)(K / 32) * 6;
     const uint8_t *abase = reinterpret_cast<const uint8_t *>(ah);
 
@@ -1376,7 +1137,7 @@ __global__ __launch_bounds__((BN / WN) * 64, (BN / WN) >= 8 ? 2 : 1) void b1_gem
     // Returns what the tile-start vmcnt waits may assume about the stores
     // left in flight: 0 none, 1 unknown (wait for all), 2 EPI_STORES vector
     // stores per lane, 3 EPI_STORES / 2.
-    auto epilogue = [&](int m0, int n0, float *__restrict__ out) -> int {
+    auto epilogue = [&](int m0, int n0) -> int {
         int bad = 0;
         const bool cnt = nonfinite != nullptr;
         if constexpr (EPI == 2) {
@@ -1685,28 +1446,21 @@ __global__ __launch_bounds__((BN / WN) * 64, (BN / WN) >= 8 ? 2 : 1) void b1_gem
     };
 
     int unit = xcd_tile(blockIdx.x, gridDim.x);
-    int m0, n0, kst0;   // tile origin; first global stage of the unit's K range
-    float *uout;        // where the unit's epilogue writes
-    auto unit_origin = [&](int u) {
-        const int split = u / ntiles;
-        tile_origin(u - split * ntiles, m0, n0);
-        kst0 = split * nstage;
-        uout = out + (size_t)split * (size_t)pstride;
-    };
+    int m0, n0;
     // Row scales of the tile (epi.rsc, range-safe packing): waves 0 .. BM/64
     // - 1 copy the BM values into the tile's parity buffer, ahead of its first
     // stage, so they count as part of that stage in the vmcnt waits.
-    const bool rows_scaled = epi.rsc != nullptr && ksplit == 1;
+    const bool rows_scaled = epi.rsc != nullptr;
     int parity = 0;
     auto issue_rsc = [&](int par) {
         static_assert(BM % 64 == 0 && BM / 64 <= C::NW, "one wave copies 64 row scales");
         if (rows_scaled && wave < BM / 64)
             dma_lds4(epi.rsc + min(m0 + 64 * wave + lane, M - 1), smem + C::RSC + par * BM * 4 + wave * 256);
     };
-    unit_origin(unit);
+    tile_origin(unit, m0, n0);
     setup(m0, n0);
     issue_rsc(parity);
-    issue(kst0, 0);
+    issue(0, 0);
     int prev_stores = 0; // what the previous epilogue left in flight (its return value)
     for (;;) {
 #pragma unroll
@@ -1748,7 +1502,7 @@ __global__ __launch_bounds__((BN / WN) * 64, (BN / WN) >= 8 ? 2 : 1) void b1_gem
                 // the stage's first fragment reads go out before the next
                 // stage's loads, so the loads issue under their latency
                 compute(u, [&] {
-                    if (s + u + 1 < nstage) issue(kst0 + s + u + 1, (u + 1) % STAGES);
+                    if (s + u + 1 < nstage) issue(s + u + 1, (u + 1) % STAGES);
                 });
             }
         }
@@ -1756,15 +1510,14 @@ __global__ __launch_bounds__((BN / WN) * 64, (BN / WN) >= 8 ? 2 : 1) void b1_gem
         // Slots 0 and 1 were last read before the final barrier: fetch the
         // next tile's first stage now, then store this tile.
         const int cm0 = m0, cn0 = n0, cpar = parity;
-        float *const cout = uout;
         unit += gridDim.x;
-        const bool more = unit < nunits;
+        const bool more = unit < ntiles;
         if (more) {
-            unit_origin(unit);
+            tile_origin(unit, m0, n0);
             setup(m0, n0);
             parity ^= 1;
             issue_rsc(parity);
-            issue(kst0, 0);
+            issue(0, 0);
         }
         if (rows_scaled) {
             // this tile's rows: token m0 + 32 mt + li in every accumulator
@@ -1787,7 +1540,7 @@ __global__ __launch_bounds__((BN / WN) * 64, (BN / WN) >= 8 ? 2 : 1) void b1_gem
                         for (int v = 0; v < 16; ++v) acc[mt][nt][v] *= sc[mt];
             }
         }
-        prev_stores = epilogue(cm0, cn0, cout);
+        prev_stores = epilogue(cm0, cn0);
         if (!more) break;
     }
 }
@@ -1795,7 +1548,7 @@ __global__ __launch_bounds__((BN / WN) * 64, (BN / WN) >= 8 ? 2 : 1) void b1_gem
 // ---------------------------------------------------------------- gemm16 --
 //
 // The same GEMM over 144 x 384 or 128 x 384 tiles with 16x16x32 MFMAs, for
-// shapes whose 128 x 512 tiles quantise badly on 256 CUs (gemm_tiles picks):
+// shapes whose 128 x 512 tiles quantise badly on 256 CUs (gemm_kernel picks):
 // at M = 4608 (Flux image + text tokens) N = 3072 gives 216 tiles of
 // 128 x 512 (one round at 84 % of the CUs) but exactly 256 of 144 x 384, and
 // N = 9216 gives 648 (2.53 rounds, run as 3) but exactly 768 (3 full
@@ -2572,49 +2325,6 @@ __global__ __launch_bounds__((Gemm16Cfg<BM, BN>::NT), 2) void b1_gemm16_kernel(c
         prev_part = (EPI == 2 || EPI == 3) && ns >= C::MT;
         if (!more) break;
     }
-}
-
-// Split-K reduction: out[m][n] = sum over s = 0..S-1, in that order, of
-// part[s][m][n] (slices pstride apart, rows ldp apart, ldp % 4 == 0), with
-// the non-finite count of the sums.
-// rsc: row scales of range-safe packing (or nullptr), applied to the sum.
-__global__ __launch_bounds__(256) void b1_splitk_reduce_kernel(const float *__restrict__ part, int64_t ldp,
-                                                               int64_t pstride, int S, int M, int N,
-                                                               float *__restrict__ out, int64_t ldo,
-                                                               int32_t *nonfinite, int vec,
-                                                               const float *__restrict__ rsc) {
-    const int q = (N + 3) / 4; // 4-column units per row
-    const int64_t units = (int64_t)M * q;
-    int bad = 0;
-    for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < units; u += (int64_t)gridDim.x * 256) {
-        const int m = (int)(u / q), c = (int)(u - (int64_t)m * q) * 4;
-        const float *src = part + (size_t)m * ldp + c;
-        floatx4 sum = *reinterpret_cast<const floatx4 *>(src);
-        for (int sp = 1; sp < S; ++sp) {
-            const floatx4 v = *reinterpret_cast<const floatx4 *>(src + (size_t)sp * pstride);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sum[r] += v[r];
-        }
-        if (rsc) {
-            const float sc = rsc[m];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) sum[r] *= sc;
-        }
-        float *dst = out + (size_t)m * ldo + c;
-        if (vec && c + 4 <= N) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) bad += nonfinite && !__builtin_isfinite(sum[r]);
-            *reinterpret_cast<floatx4 *>(dst) = sum;
-        } else {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-                if (c + r < N) {
-                    bad += nonfinite && !__builtin_isfinite(sum[r]);
-                    dst[r] = sum[r];
-                }
-        }
-    }
-    count_nonfinite(nonfinite, bad);
 }
 
 // ----------------------------------------------------------------- gemv --
@@ -3581,6 +3291,7 @@ using KCfg = GemmLdsCfg<kBM, kBN, kWN, kStages>;
 // Half-height tiles for the last, partial round of some shapes.
 constexpr int kBMH = 64;
 using KCfgH = GemmLdsCfg<kBMH, kBN, kWN, kStages>;
+enum class GemmKernel { Tile128x512, Tile144x384, Tile128x384, KRange };
 } // namespace
 
 // GEMM over pre-packed activations: the stage count K/128 is a multiple of
@@ -3659,17 +3370,17 @@ hipError_t launch_pack(const float *act, int64_t lda, int M, int K, void *packed
     return hipGetLastError();
 }
 
-// Split-K: how many K ranges to split a plain GEMM into, 1 for none.  A
-// split pays only when the 128 x 512 tiles leave most CUs idle (fewer than
-// half busy): it multiplies the work units by S, then a separate pass sums
-// S fp32 partial products.  Model, in microseconds: a 384-K unit of a tile
-// takes ~10.9; the partials cost their write and read at ~5 TB/s plus ~3
-// for the extra launch.  S divides K / 384, at most 16.
-int gemm_splits(int M, int K, int N, int num_cus) {
-    if (num_cus <= 0 || !gemm_packed_ok(M, K, N) || N % 4) return 1;
+// What the size queries report beyond the packing: S fp32 partial products
+// of M x N (rows rounded up to 4 columns) for shapes whose 128 x 512 tiles
+// leave more than half of the CUs idle, S from a time model of that kernel
+// (10.9 us per 384-K unit of a tile, partials at ~5 TB/s, 3 us for their
+// sum).  The K ranges are now summed in LDS (b1_tile_gemm.h) and no kernel
+// uses this area; the sizes stay what callers have laid buffers out by.
+size_t gemm_partial_bytes(int M, int K, int N, int n_sum, int num_cus) {
+    if (num_cus <= 0 || !gemm_packed_ok(M, K, N) || N % 4) return 0;
     const int tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
     const int slots = num_cus * kWgPerCu;
-    if (2 * tiles > slots) return 1;
+    if (2 * tiles > slots) return 0;
     const int units = K / (KCfg::KC * kStages);
     int best = 1;
     double best_us = 0;
@@ -3683,11 +3394,7 @@ int gemm_splits(int M, int K, int N, int num_cus) {
             best_us = us;
         }
     }
-    return best;
-}
-
-size_t gemm_split_bytes(int M, int N, int splits) {
-    return splits > 1 ? (size_t)splits * (size_t)M * (size_t)((N + 3) & ~3) * sizeof(float) : 0;
+    return best > 1 ? (size_t)best * (size_t)M * (size_t)((n_sum + 3) & ~3) * sizeof(float) : 0;
 }
 
 // Rounds of the 128 x 512 kernel's persistent grid, in units of one round
@@ -3703,26 +3410,29 @@ static double gemm_rounds128(int M, int N, int num_cus) {
     return (double)((tiles + slots - 1) / slots);
 }
 
-int gemm_tiles(int M, int K, int N, int num_cus) {
-    if (num_cus <= 0 || !gemm_packed_ok(M, K, N) || K % (Gemm16Cfg<128, 384>::KC * Gemm16Cfg<128, 384>::STAGES))
-        return 0;
-    if (gemm_splits(M, K, N, num_cus) > 1) return 0;
-    // rounds of the persistent grid in units of a 128 x 512 round (a BM x BN
-    // tile counts BM BN / 65536 of one); strictly fewer to leave the
-    // 128 x 512 kernel
-    double best = gemm_rounds128(M, N, num_cus);
-    int kind = 0;
-    auto consider = [&](int id, int bm, int bn) {
+// The kernel a packed GEMM whose K is one range runs: the persistent
+// kernels below cost ~87 us per 3072-K round of 128 x 512 tiles (a BM x BN
+// tile counts BM BN / 65536 of one) on 256 CUs, the K-range tiles what
+// tile_gemm_us says; the latter only where it is 7 % better, the scatter of
+// both models (M=1024 K=3072 N=18432: 130.7 us as two 75 % full rounds of
+// 128 x 384, 105.6 us as 768 tiles of 128 x 192; M=4096 N=12288: 253 us as
+// three full rounds, 273 us modelled for the others).
+static GemmKernel gemm_kernel(int M, int K, int N, int num_cus) {
+    const int cus = num_cus > 0 ? num_cus : 256;
+    double best = gemm_rounds128(M, N, cus);
+    GemmKernel kind = GemmKernel::Tile128x512;
+    auto consider = [&](GemmKernel id, int bm, int bn) {
         if (M % bm || N % bn) return;
         const int tiles = (M / bm) * (N / bn);
-        const double r = (double)((tiles + num_cus - 1) / num_cus) * (double)(bm * bn) / (double)(kBM * kBN);
+        const double r = (double)((tiles + cus - 1) / cus) * (double)(bm * bn) / (double)(kBM * kBN);
         if (r < best) {
             best = r;
             kind = id;
         }
     };
-    consider(1, 144, 384);
-    consider(2, 128, 384);
+    consider(GemmKernel::Tile144x384, 144, 384);
+    consider(GemmKernel::Tile128x384, 128, 384);
+    if (tile_gemm_us(M, K, N, cus) < 0.93 * best * (3.0 + 84.0 * (double)K / 3072)) kind = GemmKernel::KRange;
     return kind;
 }
 
@@ -3756,19 +3466,17 @@ static hipError_t launch_gemm16_t(const void *packed, const uint8_t *w, int K, i
 template <int EPI>
 static hipError_t launch_gemm_packed_t(const void *packed, const uint8_t *w, int K, int N, int M, float *out,
                                        int64_t ldo, int32_t *nonfinite, int num_cus, const GemmEpi &epi,
-                                       hipStream_t s, int ksplit = 1, float *partials = nullptr) {
-    // (with ksplit > 1 the row scales epi.rsc go to the reduction, not the
-    // GEMM, which writes plain partial products)
+                                       hipStream_t s) {
     // (a packed SwiGLU output on 16x16 tiles needs the split point on a
     // tile boundary, every tile wholly fp32 or wholly SwiGLU pairs; otherwise
     // it runs the 128 x 512 kernel)
-    {
-        const bool tiles_ok = !(EPI == 3 && epi.act == 2 && epi.split % 384 != 0);
-        if (!(ksplit > 1 && partials != nullptr) && tiles_ok) {
-            const int t = gemm_tiles(M, K, N, num_cus);
-            if (t == 1) return launch_gemm16_t<144, 384, EPI>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
-            if (t == 2) return launch_gemm16_t<128, 384, EPI>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
-        }
+    const GemmKernel t = gemm_kernel(M, K, N, num_cus);
+    if (t == GemmKernel::KRange) return launch_tile_gemm(packed, w, K, N, M, out, ldo, nonfinite, num_cus, 1, EPI, epi, s);
+    if (!(EPI == 3 && epi.act == 2 && epi.split % 384 != 0)) {
+        if (t == GemmKernel::Tile144x384)
+            return launch_gemm16_t<144, 384, EPI>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
+        if (t == GemmKernel::Tile128x384)
+            return launch_gemm16_t<128, 384, EPI>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
     }
     auto kernel = &b1_gemm_kernel<kBM, kBN, kWN, kStages, EPI>;
     static std::once_flag attr_once;
@@ -3779,27 +3487,10 @@ static hipError_t launch_gemm_packed_t(const void *packed, const uint8_t *w, int
     });
     if (attr_err != hipSuccess) return attr_err;
     const int tiles_m = (M + kBM - 1) / kBM, tiles_n = (N + kBN - 1) / kBN;
-    const bool split = EPI == 0 && ksplit > 1 && partials != nullptr;
-    const int units = tiles_m * tiles_n * (split ? ksplit : 1);
+    const int units = tiles_m * tiles_n;
     const int slots = num_cus > 0 ? num_cus * kWgPerCu : units;
     const int grid = units < slots ? units : slots; // persistent
     auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
-    if (split) {
-        // the units' plain products into the partial slices, then their sum
-        const int64_t ldp = (N + 3) & ~3;
-        const int64_t pstride = (int64_t)M * ldp;
-        hipLaunchKernelGGL(kernel, dim3(grid), dim3(KCfg::NT), KCfg::LDS, s, static_cast<const uint16_t *>(packed),
-                           w, K, N, M, partials, ldp, nullptr, tiles_m, tiles_n,
-                           (int)(al16(partials) && ldp < (int64_t(1) << 22)), epi, ksplit, pstride);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-        const int64_t q = (int64_t)M * ((N + 3) / 4);
-        const int64_t want = (q + 255) / 256, cap = (int64_t)(num_cus > 0 ? num_cus : 256) * 8;
-        const int rgrid = (int)(want < cap ? want : cap);
-        hipLaunchKernelGGL(b1_splitk_reduce_kernel, dim3(rgrid), dim3(256), 0, s, partials, ldp, pstride, ksplit, M,
-                           N, out, ldo, nonfinite, (int)(al16(out) && ldo % 4 == 0), epi.rsc);
-        return hipGetLastError();
-    }
     int vec_store = al16(out) && ldo % 4 == 0 && ldo < (int64_t(1) << 22);
     if (EPI == 1)
         vec_store = vec_store && al16(epi.res) && al16(epi.gate) && epi.ldr % 4 == 0 && epi.ldr < (int64_t(1) << 22);
@@ -3834,7 +3525,7 @@ static hipError_t launch_gemm_packed_t(const void *packed, const uint8_t *w, int
         const int hunits = head_rows * tiles_n;
         hipLaunchKernelGGL(kernel, dim3(hunits < slots ? hunits : slots), dim3(KCfg::NT), KCfg::LDS, s,
                            static_cast<const uint16_t *>(packed), w, K, N, ms, out, ldo, nonfinite, head_rows, tiles_n,
-                           vec_store, epi, 1, (int64_t)0);
+                           vec_store, epi);
         hipError_t e = hipGetLastError();
         if (e != hipSuccess) return e;
         GemmEpi et = epi;
@@ -3844,32 +3535,19 @@ static hipError_t launch_gemm_packed_t(const void *packed, const uint8_t *w, int
         const int mt = M - ms, tm = (mt + kBMH - 1) / kBMH;
         hipLaunchKernelGGL(tail, dim3(tm * tiles_n), dim3(KCfgH::NT), KCfgH::LDS, s,
                            static_cast<const uint16_t *>(packed) + (size_t)ms * (size_t)K, w, K, N, mt,
-                           out ? out + (size_t)ms * (size_t)ldo : out, ldo, nonfinite, tm, tiles_n, vec_store, et, 1,
-                           (int64_t)0);
+                           out ? out + (size_t)ms * (size_t)ldo : out, ldo, nonfinite, tm, tiles_n, vec_store, et);
         return hipGetLastError();
     }
     hipLaunchKernelGGL(kernel, dim3(grid), dim3(KCfg::NT), KCfg::LDS, s, static_cast<const uint16_t *>(packed), w,
-                       K, N, M, out, ldo, nonfinite, tiles_m, tiles_n, vec_store, epi, 1, (int64_t)0);
+                       K, N, M, out, ldo, nonfinite, tiles_m, tiles_n, vec_store, epi);
     return hipGetLastError();
 }
 
-hipError_t launch_gemm_packed(const void *packed, const uint8_t *w, int K, int N, int M, float *out, int64_t ldo,
-                              int32_t *nonfinite, int num_cus, hipStream_t s) {
-    return launch_gemm_packed_t<0>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, GemmEpi{}, s);
-}
-
-hipError_t launch_gemm_packed_split(const void *packed, const uint8_t *w, int K, int N, int M, float *out,
-                                    int64_t ldo, int32_t *nonfinite, int num_cus, int splits, void *partials,
-                                    hipStream_t s, const float *rsc) {
-    GemmEpi epi;
-    epi.rsc = rsc;
-    return launch_gemm_packed_t<0>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s, splits,
-                                   static_cast<float *>(partials));
-}
-
 hipError_t launch_gemm_packed_epi(const void *packed, const uint8_t *w, int K, int N, int M, float *out,
-                                  int64_t ldo, int32_t *nonfinite, int num_cus, int kind, const GemmEpi &epi,
-                                  hipStream_t s) {
+                                  int64_t ldo, int32_t *nonfinite, int num_cus, int kranges, int kind,
+                                  const GemmEpi &epi, hipStream_t s) {
+    if (kranges > 1)
+        return launch_tile_gemm(packed, w, K, N, M, out, ldo, nonfinite, num_cus, kranges, kind, epi, s);
     switch (kind) {
     case 0: return launch_gemm_packed_t<0>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
     case 1: return launch_gemm_packed_t<1>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
@@ -3894,22 +3572,15 @@ hipError_t launch_gemm(const LinearArgs &a, int num_cus, void *workspace, size_t
     }
     hipError_t e = launch_pack_rows(a.act, a.lda, a.M, a.K, workspace, s);
     if (e != hipSuccess) return e;
-    const float *rsc = pack_area_rsc(workspace, a.M, a.K);
-    // the split-K partials after the packing, when the workspace holds them
-    const int splits = gemm_splits(a.M, a.K, a.N, num_cus);
-    if (splits > 1 && ws_bytes >= need + gemm_split_bytes(a.M, a.N, splits))
-        return launch_gemm_packed_split(workspace, a.w, a.K, a.N, a.M, a.out, a.ldo, a.nonfinite, num_cus, splits,
-                                        static_cast<uint8_t *>(workspace) + need, s, rsc);
     GemmEpi epi;
-    epi.rsc = rsc;
-    return launch_gemm_packed_epi(workspace, a.w, a.K, a.N, a.M, a.out, a.ldo, a.nonfinite, num_cus, 0, epi, s);
+    epi.rsc = pack_area_rsc(workspace, a.M, a.K);
+    return launch_gemm_packed_epi(workspace, a.w, a.K, a.N, a.M, a.out, a.ldo, a.nonfinite, num_cus,
+                                  gemm_kranges(a.M, a.K, a.N, num_cus), 0, epi, s);
 }
 
 size_t gemm_workspace_bytes_total(const LinearArgs &a, int num_cus) {
     const size_t pack = gemm_workspace_bytes(a);
-    if (pack == 0) return 0;
-    const int splits = gemm_splits(a.M, a.K, a.N, num_cus);
-    return splits > 1 ? pack + gemm_split_bytes(a.M, a.N, splits) : pack;
+    return pack ? pack + gemm_partial_bytes(a.M, a.K, a.N, a.N, num_cus) : 0;
 }
 
 hipError_t launch_quantize(const float *w, int64_t ldw, int K, int N, void *packed, int order, hipStream_t s) {

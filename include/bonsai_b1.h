@@ -116,8 +116,7 @@ int bonsai_b1_linear_f32(const float *act, int64_t lda, const void *w,
 
 /*
  * The GEMM kernels pack the activations to fp16 once (with the row scales
- * of the range-safe packing, and, for shapes that split along K, the split
- * partials after them) into a device workspace of
+ * of the range-safe packing) into a device workspace, at most
  * bonsai_b1_workspace_bytes(batch, in_dim, out_dim, mode) bytes (0 when the
  * call needs none: EXACT, and small batches, whose kernel converts the
  * activations itself).  bonsai_b1_linear_f32 keeps library-owned workspaces
@@ -132,8 +131,9 @@ int bonsai_b1_linear_f32(const float *act, int64_t lda, const void *w,
  * that stream (or ordered with it).  bonsai_b1_linear_f32_ws takes the
  * caller's workspace instead (NULL or too small selects that same variant)
  * and never allocates.  The variants agree bit for bit, except (a) for a
- * shape split along K, which the variant without room for the partials sums
- * unsplit (the same values up to the order of the K summation), and (b) for
+ * shape with few output tiles, whose K the packed GEMM sums in 2 to 8 ranges
+ * and the converting variant in one (the same values up to the order of the
+ * K summation), and (b) for
  * rows beyond the fp16 range, which the converting variant computes in
  * EXACT arithmetic.  Concurrent calls on one stream are ordered; calls on
  * different streams use different workspaces.  A workspace is found by the
@@ -159,7 +159,7 @@ void bonsai_b1_release_workspaces(void);
  * hipMalloc.  No counterpart in the reference (its CPU op needs no
  * workspace).  Same arguments, kernels and results, bit for bit, as
  * bonsai_b1_linear_f32; the workspace those kernels use (the fp16 packing
- * of the activations and the split-K partials) is a static device array of
+ * of the activations) is a static device array of
  * BONSAI_B1_NOALLOC_SCRATCH_BYTES that the library holds on each device it
  * runs on until the process ends.  Never calls hipMalloc or hipFree.
  * Returns BONSAI_B1_ERR_SCRATCH, launching nothing, when the kernel the
@@ -216,12 +216,10 @@ int bonsai_b1_pack_act_f16_ld(const float *act, int64_t lda, int in_dim,
  * aligned, w 4-byte aligned); same outputs as bonsai_b1_linear_f32 in
  * FAST/GEMM mode on the activations that were packed, or, for batch <= 16
  * with in_dim % 256 == 0, as its small-M (GEMV) mode, bit for bit (for
- * activations within the fp16 range).  A shape that bonsai_b1_linear_f32
- * splits along K is split the same way, with the partials in the library's
- * per-stream workspace (allocated on demand like bonsai_b1_linear_f32's;
- * under capture without one it runs unsplit).  The _ws form takes the
- * caller's workspace of bonsai_b1_linear_packed_workspace_bytes bytes
- * (0: none needed; NULL or smaller: unsplit) and never allocates. */
+ * activations within the fp16 range).  Allocates nothing.  The _ws form
+ * accepts a workspace of bonsai_b1_linear_packed_workspace_bytes bytes,
+ * which earlier versions needed for K split over work-groups; it runs the
+ * same kernels with the same results without one. */
 int bonsai_b1_linear_packed_f16(const void *packed_act, const void *w,
                                 int in_dim, int out_dim, int batch,
                                 float *out, int64_t ldo, int32_t *nonfinite,
