@@ -43,7 +43,6 @@ namespace {
 // ---------------------------------------------------------------- exact --
 
 constexpr int kExTN = 256; // output columns per work-group (one per thread)
-constexpr int kExKC = 256; // K staged in LDS per pass
 
 // EXACT mode: every output in the reference's scalar order
 // (src/b1_0_kernel.h:253-277): block_sum takes +-a over the block's 32
@@ -51,61 +50,122 @@ constexpr int kExKC = 256; // K staged in LDS per pass
 // an fp32 add, no contraction).  Each +-a step is fma(a, s, block_sum) with
 // s = +-1.0: the product is exact, so the fma rounds once, exactly as the
 // add or the subtract does, to the same value (signed zeros included; a
-// NaN may carry another payload).  The 32 signs of a block are formed once
-// (a shift and a bit op each) for the work-group's TM rows, which share
-// them: about 1 + 2 / TM VALU operations per multiply-accumulate, where a
-// select between a and -a and an add made 2 + 2 / TM.
-template <int TM>
+// NaN may carry another payload).
+//
+// What bounds it: the one FMA a multiply-accumulate needs, 1.8 ns a wave
+// instruction per SIMD (66 us at M=256 K=3072 N=3072), so the rest is kept
+// off the VALU.  The activations are the same in all lanes: they come by
+// scalar loads, KS elements of the TM rows a step, one step ahead, and enter
+// the FMA as its SGPR operand (as LDS broadcasts the reads were the bound:
+// 16 bytes a lane for 4 FMAs).  The signs are fp16 +-1.0 pairs (elements d
+// and d + 16), a shift and a bit op for two, read as halves by
+// v_fma_mix_f32, which converts them exactly and runs at the FMA's rate.
+// The packed weights arrive 24 bytes (4 blocks) at a time, one ahead.  Each
+// XCD takes a contiguous run of row groups, so that the scalar loads' lines
+// are in its L2, and vector loads touch the rows' lines well ahead of them.
+// M=256 K=3072 N=3072: with LDS broadcasts and fp32 signs 153 us; this form
+// on repeated inputs 115 in grid order, 94 by XCD; on new inputs each call
+// 124 without the early touch, 109 with it.
+template <int TM, int KS>
 __global__ __launch_bounds__(kExTN) void b1_exact_kernel(LinearArgs p) {
 #pragma clang fp contract(off)
-    __shared__ __attribute__((aligned(16))) float As[TM][kExKC];
-    const int n = blockIdx.x * kExTN + threadIdx.x;
-    const int m0 = blockIdx.y * TM;
+    typedef float row_v __attribute__((ext_vector_type(KS), aligned(4)));
+    typedef const __attribute__((address_space(4))) char const_u8; // scalar loads
+    typedef const __attribute__((address_space(4))) row_v const_row;
+    const int cols = gridDim.x;
+    const int t = xcd_tile((int)(blockIdx.x + blockIdx.y * gridDim.x), (int)(gridDim.x * gridDim.y));
+    const int m0 = t / cols * TM, n = t % cols * kExTN + threadIdx.x;
     const int nb = p.K / 32;
-    const int nrow = n < p.N ? n : p.N - 1;
-    const uint16_t *wr = reinterpret_cast<const uint16_t *>(p.w + (size_t)nrow * nb * 6);
+    const uint8_t *wr = p.w + (size_t)(n < p.N ? n : p.N - 1) * nb * 6;
+    // Row pointers (rows past M read the last one).  The empty asm keeps the
+    // compiler from recomputing them from the row stride, and the step's
+    // offset (below) from merging or hoisting loads of several steps: both
+    // overflow the scalar registers.
+    uint64_t row[TM];
+#pragma unroll
+    for (int r = 0; r < TM; ++r) {
+        row[r] = reinterpret_cast<uint64_t>(p.act + (size_t)min(m0 + r, p.M - 1) * p.lda);
+        asm volatile("" : "+s"(row[r]));
+    }
+    auto advance = [&](uint32_t bytes) {
+#pragma unroll
+        for (int r = 0; r < TM; ++r) {
+            row[r] += bytes;
+            asm volatile("" : "+s"(row[r]));
+        }
+    };
+    row_v next[TM];
+    auto load = [&](uint32_t off) {
+        asm volatile("" : "+s"(off));
+#pragma unroll
+        for (int r = 0; r < TM; ++r) next[r] = *(const_row *)((const_u8 *)row[r] + off);
+    };
     float sum[TM];
 #pragma unroll
     for (int r = 0; r < TM; ++r) sum[r] = 0.0f;
-
-    for (int kc = 0; kc < p.K; kc += kExKC) {
-        const int klen = min(kExKC, p.K - kc);
-        __syncthreads();
-        for (int i = threadIdx.x; i < TM * kExKC; i += kExTN) {
-            const int r = i / kExKC, c = i - r * kExKC;
-            As[r][c] = (m0 + r < p.M && c < klen)
-                           ? p.act[(size_t)(m0 + r) * p.lda + kc + c]
-                           : 0.0f;
-        }
-        __syncthreads();
-        const int nbk = klen / 32;
-        for (int b = 0; b < nbk; ++b) {
-            const uint16_t *blk = wr + (size_t)(kc / 32 + b) * 3;
-            const float scale = (float)__builtin_bit_cast(_Float16, blk[0]);
-            const uint32_t bits = (uint32_t)blk[1] | ((uint32_t)blk[2] << 16);
-            float bs[TM];
+    // one block, `off` bytes past the row pointers; its last step loads the
+    // first of the block at off_next
+    auto block = [&](uint32_t bits, float scale, uint32_t off, uint32_t off_next) {
+        float bs[TM];
 #pragma unroll
-            for (int r = 0; r < TM; ++r) bs[r] = 0.0f;
+        for (int r = 0; r < TM; ++r) bs[r] = 0.0f;
 #pragma unroll
-            for (int i4 = 0; i4 < 8; ++i4) {
+        for (int i0 = 0; i0 < 32; i0 += KS) {
+            // scalar loads return out of order: wait for this step's before
+            // the next step's are issued
+            wait_lgkmcnt0();
+            __builtin_amdgcn_sched_barrier(0);
+            row_v a[TM];
+#pragma unroll
+            for (int r = 0; r < TM; ++r) a[r] = next[r];
+            load(i0 + KS < 32 ? off + 4 * (i0 + KS) : off_next);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < KS; ++j) {
+                const int i = i0 + j;
                 // +1.0 for a set bit, -1.0 for a clear one
-                float sg[4];
+                const half2v sg = __builtin_bit_cast(half2v, ((bits << (15 - (i & 15))) & kSignPair) ^ 0xBC00BC00u);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int i = 4 * i4 + j;
-                    sg[j] = __builtin_bit_cast(float, ((bits << (31 - i)) & 0x80000000u) ^ 0xBF800000u);
-                }
-#pragma unroll
-                for (int r = 0; r < TM; ++r) {
-                    const floatx4 a = *reinterpret_cast<const floatx4 *>(&As[r][b * 32 + 4 * i4]);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) bs[r] = __builtin_fmaf(a[j], sg[j], bs[r]);
-                }
+                for (int r = 0; r < TM; ++r) bs[r] = __builtin_fmaf(a[r][j], (float)sg[i >> 4], bs[r]);
             }
-#pragma unroll
-            for (int r = 0; r < TM; ++r) sum[r] = sum[r] + scale * bs[r];
+            __builtin_amdgcn_sched_barrier(0);
         }
+#pragma unroll
+        for (int r = 0; r < TM; ++r) sum[r] = sum[r] + scale * bs[r];
+    };
+    auto half_lo = [](uint32_t d) { return (float)__builtin_bit_cast(_Float16, (uint16_t)d); };
+    // Touches one 128-byte line of a row a lane, `line` lines into it, so
+    // that it is in L2 when the scalar loads reach it: 64 / TM lines at the
+    // start, then the 4 of the quad as far ahead.
+    auto touch = [&](int r, int line, bool mine) {
+        float v = 0.0f;
+        if (mine && line * 32 < p.K) v = p.act[(size_t)min(m0 + r, p.M - 1) * p.lda + line * 32];
+        return v;
+    };
+    constexpr int AHEAD = 64 / TM;
+    float warm = touch(threadIdx.x / AHEAD, threadIdx.x % AHEAD, threadIdx.x < 64);
+    load(0);
+    const int quads = nb / 4;
+    uint32_t q[6], qn[6];
+    if (quads) __builtin_memcpy(qn, wr, 24);
+    for (int c = 0; c < quads; ++c) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) q[i] = qn[i];
+        asm volatile("" ::"v"(warm));
+        warm = touch(threadIdx.x >> 2, AHEAD + 4 * c + (threadIdx.x & 3), threadIdx.x < 4 * TM);
+        __builtin_memcpy(qn, wr + (size_t)(c + 1 < quads ? c + 1 : 0) * 24, 24);
+        block(__builtin_amdgcn_alignbit(q[1], q[0], 16), half_lo(q[0]), 0, 128);
+        block(q[2], half_lo(q[1] >> 16), 128, 256);
+        block(__builtin_amdgcn_alignbit(q[4], q[3], 16), half_lo(q[3]), 256, 384);
+        block(q[5], half_lo(q[4] >> 16), 384, 4 * c + 4 < nb ? 512 : 0);
+        advance(512);
     }
+    for (int b = 4 * quads; b < nb; ++b) {
+        const uint16_t *blk = reinterpret_cast<const uint16_t *>(wr + (size_t)b * 6);
+        block((uint32_t)blk[1] | (uint32_t)blk[2] << 16, half_lo(blk[0]), 0, b + 1 < nb ? 128 : 0);
+        advance(128);
+    }
+    asm volatile("" ::"v"(warm));
     if (n >= p.N) return;
     int bad = 0;
 #pragma unroll
@@ -3257,21 +3317,28 @@ __global__ __launch_bounds__(kGvWaves * 64, WL == kG4WL2 ? 4 : 2) void b1_gemv_g
 // ------------------------------------------------------------- launchers --
 
 hipError_t launch_exact(const LinearArgs &a, int num_cus, hipStream_t s) {
-    // rows a work-group shares its signs over: 16 or 8 while that leaves
-    // at least 4 work-groups (16 waves) a CU, else 4 (a small grid needs
-    // the work-groups more than the shared signs)
-    const int64_t cols = (a.N + kExTN - 1) / kExTN;
-    const int64_t want = 4 * (int64_t)(num_cus > 0 ? num_cus : 256);
+    // Rows TM a work-group shares its signs over: 4, 2 or 1.  A launch takes
+    // about q work-groups a CU (rounded up) times what one adds to a busy CU,
+    // or what one takes alone if that is longer; us at K = 3072: TM = 4 31.5
+    // and 38 (q = 3, M=256 N=3072: 94), TM = 2 17.4 and 22, TM = 1 11.8 and
+    // 15 (q = 1, M=7 N=3072: 15.1, against 22 with TM = 2 and 38 with 4).
+    const int64_t cus = num_cus > 0 ? num_cus : 256, cols = (a.N + kExTN - 1) / kExTN;
+    auto us = [&](int tm, double add, double alone) {
+        const int64_t wgs = cols * ((a.M + (int64_t)tm - 1) / tm);
+        const double busy = (double)((wgs + cus - 1) / cus) * add;
+        return busy > alone ? busy : alone;
+    };
+    const double us1 = us(1, 11.8, 15.0), us2 = us(2, 17.4, 22.0), us4 = us(4, 31.5, 38.0);
     auto go = [&](auto kernel, int tm) {
-        const dim3 grid((unsigned)cols, (unsigned)((a.M + tm - 1) / tm));
+        const dim3 grid((unsigned)cols, (unsigned)((a.M + (int64_t)tm - 1) / tm));
         hipLaunchKernelGGL(kernel, grid, dim3(kExTN), 0, s, a);
     };
-    if (a.M > 8 && cols * ((a.M + 15) / 16) >= want)
-        go(b1_exact_kernel<16>, 16);
-    else if (a.M > 4 && cols * ((a.M + 7) / 8) >= want)
-        go(b1_exact_kernel<8>, 8);
+    if (us1 <= us2 && us1 <= us4)
+        go(b1_exact_kernel<1, 32>, 1);
+    else if (us2 <= us4)
+        go(b1_exact_kernel<2, 16>, 2);
     else
-        go(b1_exact_kernel<4>, 4);
+        go(b1_exact_kernel<4, 8>, 4);
     return hipGetLastError();
 }
 
