@@ -47,7 +47,7 @@ hipError_t launch_exact(const LinearArgs &a, int num_cus, hipStream_t s);
 // With a workspace of gemm_workspace_bytes(a) bytes (> 0 when K % 384 == 0)
 // the activations are packed to fp16 once (range-safe, launch_pack_rows)
 // and streamed into LDS directly; otherwise the kernel converts them while
-// staging each tile, and launch_fixup_rows follows.
+// staging each tile and computes rows beyond the fp16 range exactly itself.
 bool gemm_supported(const LinearArgs &a);
 size_t gemm_workspace_bytes(const LinearArgs &a);
 // The size callers are told: the packing and the area gemm_partial_bytes

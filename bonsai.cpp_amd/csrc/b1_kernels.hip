@@ -194,10 +194,26 @@ struct GemmCfg {
     static_assert(WM % 32 == 0 && WN % 32 == 0, "32x32 sub-tiles");
 };
 
+// The GEMM that converts fp32 activations while it stages each tile, for
+// calls without a packing (no workspace, or K no multiple of 384).  A tile
+// reads its rows once per column tile and its weights once per row tile, 4
+// bytes an activation, so wide tiles suit many tokens; with few, a tile's
+// serial K loop is what takes the time and small tiles fill the CUs
+// (launch_fused picks).  Every tile sums K in the same order: the same bits.
+// us with 128 x 512 tiles only -> now: M=1000 K=2048 N=5504 58.8 -> 40.2,
+// M=77 K=2048 N=5504 50 -> 21 (kernel alone).
+//
+// A row holding an |a| >= 65520 (or an inf), which fp16 cannot take, is not
+// stored from the tile: the work-group, which has seen all of the row,
+// computes its columns in the reference's scalar order, the arithmetic of
+// b1_exact_kernel, so its outputs are EXACT mode's bit for bit.  (A second
+// launch that read every row again to find them took 5 us at M=1000.)
 template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kernel(LinearArgs p, int tiles_n) {
     using C = GemmCfg<BM, BN, WM, WN>;
     __shared__ __attribute__((aligned(16))) uint8_t lds[2 * C::STAGE];
+    __shared__ uint32_t over[BM]; // rows beyond the fp16 range
+    static_assert(BM <= C::NT, "one thread a row clears the flags");
 
     const int t = xcd_tile(blockIdx.x, gridDim.x);
     const int tm = t / tiles_n, tn = t - tm * tiles_n;
@@ -227,6 +243,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kern
             }
         }
     };
+    float amax[C::UPT]; // largest magnitude of the unit's row and quad
+#pragma unroll
+    for (int u = 0; u < C::UPT; ++u) amax[u] = 0.0f;
+    if (tid < BM) over[tid] = 0; // (set after the last stage)
     auto store_a = [&](int buf) {
 #pragma unroll
         for (int u = 0; u < C::UPT; ++u) {
@@ -234,7 +254,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kern
             const int c = id & 3, blk = (id >> 2) & 1, row = id >> 3;
             u32x4 v;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] = pack_f16(ar[u][0][j], ar[u][1][j]);
+            for (int j = 0; j < 4; ++j) {
+                amax[u] = absmax3(amax[u], ar[u][0][j], ar[u][1][j]);
+                v[j] = pack_f16(ar[u][0][j], ar[u][1][j]);
+            }
             *reinterpret_cast<u32x4 *>(lds + buf * C::STAGE + row * C::ROW + blk * 64 + c * 16) = v;
         }
     };
@@ -282,6 +305,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kern
                 }
                 wg[nt] = wd >> (4 * g);
             }
+            // pairs 0 .. 3 (h = 0) and 8 .. 11 of the shifted word
+            u32x4 wb[C::NTL][2];
+#pragma unroll
+            for (int nt = 0; nt < C::NTL; ++nt) wpair_quads<0>(wg[nt], wg[nt] >> 8, s2[nt], wb[nt][0], wb[nt][1]);
 #pragma unroll
             for (int h = 0; h < 2; ++h) {
                 half8 af[C::MT];
@@ -290,10 +317,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kern
                     af[mt] = *reinterpret_cast<const half8 *>(base + mt * 32 * C::ROW + b * 64 + h * 32);
 #pragma unroll
                 for (int nt = 0; nt < C::NTL; ++nt) {
-                    u32x4 bd;
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) bd[j] = wpair(wg[nt], 15 - 8 * h - j, s2[nt]);
-                    const half8 bf = __builtin_bit_cast(half8, bd);
+                    const half8 bf = __builtin_bit_cast(half8, wb[nt][h]);
 #pragma unroll
                     for (int mt = 0; mt < C::MT; ++mt)
                         acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], bf, acc[mt][nt], 0, 0, 0);
@@ -326,7 +350,14 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kern
 
     // ---- epilogue: 32x32 accumulator layout: lane column li, rows
     // 8*(v/4) + 4*g + v%4 of each sub-tile ------------------------------
-    int bad = 0;
+    int bad = 0, mine = 0;
+#pragma unroll
+    for (int u = 0; u < C::UPT; ++u)
+        if (amax[u] >= kF16Overflow) {
+            over[(tid + u * C::NT) >> 3] = 1;
+            mine = 1;
+        }
+    const int any = __syncthreads_or(mine);
 #pragma unroll
     for (int mt = 0; mt < C::MT; ++mt) {
 #pragma unroll
@@ -335,12 +366,35 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kern
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int m = m0 + wm * WM + mt * 32 + 8 * (v >> 2) + 4 * g + (v & 3);
-                if (m < p.M && n < p.N) {
+                if (m < p.M && n < p.N && !(any && over[m - m0])) {
                     const float y = acc[mt][nt][v];
                     bad += !__builtin_isfinite(y);
                     p.out[(size_t)m * p.ldo + n] = y;
                 }
             }
+        }
+    }
+    if (any) {
+#pragma clang fp contract(off)
+        for (int e = tid; e < BM * BN; e += C::NT) {
+            const int r = e / BN, m = m0 + r, n = n0 + e - r * BN;
+            if (!over[r] || m >= p.M || n >= p.N) continue;
+            const float *xr = p.act + (size_t)m * p.lda;
+            const uint16_t *wr = reinterpret_cast<const uint16_t *>(p.w + (size_t)n * rs);
+            float sum = 0.0f;
+            for (int b = 0; b < p.K / 32; ++b) {
+                const float scale = (float)__builtin_bit_cast(_Float16, wr[3 * b]);
+                const uint32_t bits = (uint32_t)wr[3 * b + 1] | ((uint32_t)wr[3 * b + 2] << 16);
+                float bs = 0.0f;
+                for (int i4 = 0; i4 < 32; i4 += 4) {
+                    const floatx4 a = *reinterpret_cast<const floatx4 *>(xr + 32 * b + i4);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) bs = ((bits >> (i4 + j)) & 1u) ? bs + a[j] : bs - a[j];
+                }
+                sum = sum + scale * bs;
+            }
+            bad += !__builtin_isfinite(sum);
+            p.out[(size_t)m * p.ldo + n] = sum;
         }
     }
     count_nonfinite(p.nonfinite, bad);
@@ -790,9 +844,8 @@ __global__ __launch_bounds__(256) void b1_pack_rows_kernel(const float *__restri
     }
 }
 
-// Exact recomputation of the rows that the paths converting fp32
-// activations inside their own kernel (the fused-conversion GEMM and the
-// small-M kernels, used without a workspace) cannot take in fp16: a row
+// Exact recomputation of the rows that the small-M kernel of K % 256 != 0,
+// which converts fp32 activations itself, cannot take in fp16: a row
 // holding an |a| >= 65520 (or an inf) is computed again in the reference's
 // scalar order, the arithmetic of b1_exact_kernel, so its outputs are
 // EXACT mode's bit for bit.  One work-group per row; other rows only cost a
@@ -3624,18 +3677,39 @@ hipError_t launch_gemm_packed_epi(const void *packed, const uint8_t *w, int K, i
     }
 }
 
+// The fused-conversion GEMM's tile by a time model: a launch of q tiles a CU
+// (rounded up) takes q times what one adds to a busy CU per 64 of K, or what
+// one takes alone if that is longer.  us per 64 of K, measured over 17 to
+// 4096 tokens: 128 x 512 2.65 and 1.9, 64 x 256 0.80 and 0.95, 64 x 128 0.47
+// and 0.75, 32 x 64 0.19 and 0.58 (M=4096 K=2048 N=8192: 172 us with 128 x
+// 512, 208 with 64 x 256, 243 with 64 x 128; M=1000 N=5504: 61, 41 and 40;
+// M=300 K=4096 N=1027: 100, 53, 44, and 34 with 32 x 64).
+static hipError_t launch_fused(const LinearArgs &a, int num_cus, hipStream_t s) {
+    const int64_t cus = num_cus > 0 ? num_cus : 256;
+    auto tiles = [&](int bm, int bn) {
+        return ((a.M + (int64_t)bm - 1) / bm) * ((a.N + (int64_t)bn - 1) / bn);
+    };
+    auto us = [&](int bm, int bn, double add, double alone) {
+        const double busy = (double)((tiles(bm, bn) + cus - 1) / cus) * add;
+        return busy > alone ? busy : alone;
+    };
+    const double t512 = us(128, 512, 2.65, 1.9), t256 = us(64, 256, 0.80, 0.95), t128 = us(64, 128, 0.47, 0.75),
+                 t64 = us(32, 64, 0.19, 0.58);
+    auto go = [&](auto kernel, int bm, int bn, int threads) {
+        hipLaunchKernelGGL(kernel, dim3((unsigned)tiles(bm, bn)), dim3(threads), 0, s, a, (a.N + bn - 1) / bn);
+        return hipGetLastError();
+    };
+    if (t512 <= t256 && t512 <= t128 && t512 <= t64) return go(b1_gemm_fused_kernel<128, 512, 128, 64>, 128, 512, 512);
+    if (t256 <= t128 && t256 <= t64) return go(b1_gemm_fused_kernel<64, 256, 64, 64>, 64, 256, 256);
+    if (t128 <= t64) return go(b1_gemm_fused_kernel<64, 128, 64, 32>, 64, 128, 256);
+    return go(b1_gemm_fused_kernel<32, 64, 32, 32>, 32, 64, 128);
+}
+
 hipError_t launch_gemm(const LinearArgs &a, int num_cus, void *workspace, size_t ws_bytes, hipStream_t s) {
     const size_t need = gemm_workspace_bytes(a);
     if (need == 0 || workspace == nullptr || ws_bytes < need) {
-        // Fused-conversion kernel: no workspace needed; rows its fp16
-        // conversion overflows are then computed exactly.
-        constexpr int BM = 128, BN = 512, WM = 128, WN = 64;
-        using C = GemmCfg<BM, BN, WM, WN>;
-        const int tiles_m = (a.M + BM - 1) / BM, tiles_n = (a.N + BN - 1) / BN;
-        hipLaunchKernelGGL((b1_gemm_fused_kernel<BM, BN, WM, WN>), dim3(tiles_m * tiles_n), dim3(C::NT), 0, s, a,
-                           tiles_n);
-        const hipError_t e = hipGetLastError();
-        return e == hipSuccess ? launch_fixup_rows(a, s) : e;
+        // Fused-conversion kernel: no workspace needed
+        return launch_fused(a, num_cus, s);
     }
     hipError_t e = launch_pack_rows(a.act, a.lda, a.M, a.K, workspace, s);
     if (e != hipSuccess) return e;

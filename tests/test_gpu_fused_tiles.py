@@ -1,0 +1,75 @@
+"""The GEMM that converts fp32 activations tile by tile (b1_gemm_fused_kernel,
+in_dim % 384 != 0 or no workspace) at every tile its launcher picks on 256 CUs,
+with row and column remainders.
+
+Bar for rows within the fp16 range: against the float64 product of the
+fp16-rounded activations, per element |y - ref| <= 2 K 2^-24 sum_k |a_k w_k|,
+the bound of an fp32 sum of K products in any order (twice, for products added
+pairwise inside an MFMA step).  Rows holding an |a| >= 65520 or an infinity:
+EXACT mode's bits; NaN rows: NaN; the non-finite counter counts what is stored.
+"""
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [  # (m, k, n), tile on 256 CUs
+    (17, 64, 1), (33, 448, 65), (77, 2048, 5504), (300, 320, 1027),   # 32 x 64
+    (1000, 256, 5500), (640, 128, 4097),                              # 64 x 128
+    (1000, 192, 8100), (1024, 64, 8193),                              # 64 x 256
+    (2000, 448, 8100), (2049, 64, 8192),                              # 128 x 512
+]
+
+
+@pytest.fixture(scope="module")
+def torch():
+    import torch as t
+    assert t.cuda.is_available(), "GPU tests need the MI355X"
+    return t
+
+
+@pytest.fixture(scope="module")
+def b1(torch):
+    import bonsai_b1
+    bonsai_b1.load()
+    return bonsai_b1
+
+
+def unpack(torch, raw, n, k):
+    blocks = raw.reshape(n, k // 32, 6)
+    scale = blocks[:, :, :2].contiguous().view(torch.float16).double()
+    bits = torch.arange(8, device=raw.device, dtype=torch.uint8)
+    sign = 2.0 * ((blocks[:, :, 2:].unsqueeze(-1) >> bits) & 1).double() - 1.0
+    return (sign.reshape(n, k // 32, 32) * scale).reshape(n, k)
+
+
+@pytest.mark.parametrize("m,k,n", SHAPES)
+def test_tiles(torch, b1, m, k, n):
+    from bonsai_b1 import synth
+    print(f"fused gemm ({m},{k},{n})", flush=True)
+    a = synth.device_activations(m, k, 51)
+    w = synth.device_packed_weights(n, k, 52)
+    buf = torch.full((m, n + 3), 7.0, device="cuda")
+    b1.linear(a, w, n, out=buf[:, :n], mode="gemm")
+    torch.cuda.synchronize()
+    y = buf[:, :n].clone()
+    assert bool((buf[:, n:] == 7.0).all())
+    h, wd = a.half().double(), unpack(torch, w, n, k)
+    ref, mag = h @ wd.t(), h.abs() @ wd.abs().t()
+    assert float(((y.double() - ref).abs() / (2.0 * k * 2.0 ** -24 * mag)).max()) <= 1.0
+    # rows beyond the fp16 range, first, last and at a tile's edge
+    big = sorted({0, min(30, m - 1), m // 2, m - 1})
+    a[big[0], k - 1] = 65520.0
+    for r in big[1:]:
+        a[r] *= 1.0e6
+    a[m - 1, 1] = float("inf")
+    a[m - 2, 2] = float("nan")
+    nf = torch.zeros(1, dtype=torch.int32, device="cuda")
+    z = b1.linear(a, w, n, mode="gemm", nonfinite=nf)
+    e = b1.linear(a, w, n, mode="exact")
+    torch.cuda.synchronize()
+    keep = torch.ones(m, dtype=torch.bool, device="cuda")
+    keep[big + [m - 2]] = False
+    assert torch.equal(z[keep], y[keep])
+    assert torch.equal(z[big], e[big])
+    assert bool(torch.isnan(z[m - 2]).all())
+    assert int(nf.item()) == int((~torch.isfinite(z)).sum())
