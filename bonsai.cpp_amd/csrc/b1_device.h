@@ -174,7 +174,7 @@ __device__ __forceinline__ uint32_t wpair(uint32_t w, int sh, uint32_t scale2) {
 // operand hazard).
 template <int SH>
 __device__ __forceinline__ uint64_t shl64(uint64_t v) {
-    static_assert(SH >= 8 && SH <= 15, "pairs d < 8");
+    static_assert(SH >= 0 && SH <= 15, "a 16-bit half");
     uint64_t r;
     asm("v_lshlrev_b64 %0, %1, %2" : "=v"(r) : "I"(SH), "v"(v));
     return r;
@@ -195,6 +195,17 @@ __device__ __forceinline__ void wpair_quads(uint32_t w, uint32_t w8, uint32_t sc
     hi[1] = xnor_sel(kSignPair, (uint32_t)(v1 >> 32), scale2);
     hi[2] = xnor_sel(kSignPair, (uint32_t)(v2 >> 32), scale2);
     hi[3] = xnor_sel(kSignPair, (uint32_t)(v3 >> 32), scale2);
+}
+
+// The weight dwords of pairs d .. d + 3 from the sign word shifted so that
+// pair d + 3's bits are at 15 and 31: one 32-bit and one 64-bit shift (the
+// bit the latter carries into its high dword is not a sign) instead of a
+// shift a pair.
+__device__ __forceinline__ u32x4 wpair4(uint32_t w, uint32_t scale2) {
+    const uint32_t w2 = w << 2;
+    const uint64_t v = shl64<1>((uint64_t)w2 << 32 | w);
+    return u32x4{xnor_sel(kSignPair, (uint32_t)(v >> 32), scale2), xnor_sel(kSignPair, w2, scale2),
+                 xnor_sel(kSignPair, (uint32_t)v, scale2), xnor_sel(kSignPair, w, scale2)};
 }
 
 __device__ __forceinline__ void count_nonfinite(int32_t *ctr, int bad) {

@@ -61,19 +61,21 @@ size_t gemm_partial_bytes(int M, int K, int N, int n_sum, int num_cus);
 
 // The number of contiguous K ranges a packed GEMM sums separately and then
 // adds in order (1, 2, 4 or 8), a function of the shape and CU count only,
-// so that every entry point and epilogue gives a linear the same bits: 1
-// when 64 x 192 tiles give at least 1.25 work-groups a CU, else as many as
-// fill the CUs with 64-row tiles of 48 (8 ranges), 96 (4) or 192 (2)
-// columns, and no range shorter than 384.  With one range every kernel of
+// so that every entry point and epilogue gives a linear the same bits: the
+// fastest by a time model of the tiles (and, for 1, of the persistent
+// kernels), no range shorter than 384, and 1 from 1.25 tiles of 64 x 192 a CU
+// on.  With one range every kernel of
 // the packed GEMM gives the same bits (the 16x16x32 and 32x32x16 MFMAs add
 // a K-slot order's products alike), so which of them runs is free.
 int gemm_kranges(int M, int K, int N, int num_cus);
-// The K-range tile GEMM (b1_tile_gemm.h), any K % 128 == 0 (K % 64 == 0 for
-// 2, 4 and 8 ranges), and its modelled time for one range in us.
+// The K-range tile GEMM (b1_tile_gemm.h), any K % 64 == 0.
 hipError_t launch_tile_gemm(const void *packed, const uint8_t *w, int K, int N, int M, float *out, int64_t ldo,
                             int32_t *nonfinite, int num_cus, int kranges, int kind, const GemmEpi &epi,
                             hipStream_t s);
-double tile_gemm_us(int M, int K, int N, int num_cus);
+// Modelled us of the K-range tiles at a number of ranges, and of the best
+// persistent kernel.
+double tile_gemm_us(int M, int K, int N, int num_cus, int kranges);
+double persistent_gemm_us(int M, int K, int N, int num_cus);
 
 // The two halves of the workspace path.  Packed activations: u32 word
 // (row m, 16 j + d) = fp16(a[m][32 j + d]) | fp16(a[m][32 j + d + 16]) << 16,

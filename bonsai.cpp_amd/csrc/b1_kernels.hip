@@ -3530,14 +3530,10 @@ static double gemm_rounds128(int M, int N, int num_cus) {
     return (double)((tiles + slots - 1) / slots);
 }
 
-// The kernel a packed GEMM whose K is one range runs: the persistent
-// kernels below cost ~87 us per 3072-K round of 128 x 512 tiles (a BM x BN
-// tile counts BM BN / 65536 of one) on 256 CUs, the K-range tiles what
-// tile_gemm_us says; the latter only where it is 7 % better, the scatter of
-// both models (M=1024 K=3072 N=18432: 130.7 us as two 75 % full rounds of
-// 128 x 384, 105.6 us as 768 tiles of 128 x 192; M=4096 N=12288: 253 us as
-// three full rounds, 273 us modelled for the others).
-static GemmKernel gemm_kernel(int M, int K, int N, int num_cus) {
+// The persistent kernel a packed GEMM takes, by rounds of the grid: ~87 us a
+// 3072-K round of 128 x 512 tiles (a BM x BN tile counts BM BN / 65536 of
+// one) on 256 CUs.
+static GemmKernel persistent_kernel(int M, int N, int num_cus, double *rounds) {
     const int cus = num_cus > 0 ? num_cus : 256;
     double best = gemm_rounds128(M, N, cus);
     GemmKernel kind = GemmKernel::Tile128x512;
@@ -3552,8 +3548,26 @@ static GemmKernel gemm_kernel(int M, int K, int N, int num_cus) {
     };
     consider(GemmKernel::Tile144x384, 144, 384);
     consider(GemmKernel::Tile128x384, 128, 384);
-    if (tile_gemm_us(M, K, N, cus) < 0.93 * best * (3.0 + 84.0 * (double)K / 3072)) kind = GemmKernel::KRange;
+    *rounds = best;
     return kind;
+}
+
+double persistent_gemm_us(int M, int K, int N, int num_cus) {
+    double rounds;
+    persistent_kernel(M, N, num_cus, &rounds);
+    return rounds * (3.0 + 84.0 * (double)K / 3072);
+}
+
+// The kernel a packed GEMM whose K is one range runs: the faster by the time
+// models of the persistent kernels and of the K-range tiles, the latter only
+// where it is 7 % better, the scatter of both models (M=1024 K=3072 N=18432:
+// 130.7 us as two 75 % full rounds of 128 x 384, 107 us as 768 tiles of 128 x
+// 192; M=4096 N=12288: 253 us as three full rounds, 300 us modelled for the
+// others).
+static GemmKernel gemm_kernel(int M, int K, int N, int num_cus) {
+    double rounds;
+    const GemmKernel kind = persistent_kernel(M, N, num_cus, &rounds);
+    return tile_gemm_us(M, K, N, num_cus, 1) < 0.93 * persistent_gemm_us(M, K, N, num_cus) ? GemmKernel::KRange : kind;
 }
 
 template <int BM, int BN, int EPI>

@@ -14,44 +14,50 @@ namespace {
 #include "b1_tile_gemm.h"
 
 // The tiles, by number of K ranges: BM x WN per wave, NWN waves along N, KG
-// ranges, KS per stage, R stages in the ring, and whether the packed-output
+// ranges, KS per stage, R stages in the ring, L pairs of a column a load, and whether the packed-output
 // epilogue can use them (whole 32-column blocks; 64 for SwiGLU pairs).
-//                 BM  WN NWN KG  KS  R
-using T8s = TileCfg<32, 48, 1, 8, 64, 3>;
-using T8 = TileCfg<64, 48, 1, 8, 64, 2>;
-using T8sp = TileCfg<32, 64, 1, 8, 64, 3>;
-using T8p = TileCfg<64, 64, 1, 8, 64, 2>;
-using T4s = TileCfg<32, 48, 2, 4, 64, 4>;
-using T4 = TileCfg<64, 48, 2, 4, 64, 4>;
-using T4p = TileCfg<64, 64, 2, 4, 64, 3>;
-using T2s = TileCfg<64, 48, 2, 2, 64, 4>;
-using T2sp = TileCfg<64, 64, 2, 2, 64, 3>;
-using T2 = TileCfg<64, 48, 4, 2, 64, 4>;
-using T1s = TileCfg<32, 48, 4, 1, 64, 4>;
-using T1 = TileCfg<64, 48, 4, 1, 128, 3>;
-using T1b = TileCfg<128, 48, 4, 1, 64, 3>;
+//                 BM  WN NWN KG  KS  R  L
+using T8s = TileCfg<32, 48, 1, 8, 64, 2, 4>;
+using T8 = TileCfg<64, 48, 1, 8, 64, 2, 1>;
+using T8sp = TileCfg<32, 64, 1, 8, 64, 3, 2>;
+using T8p = TileCfg<64, 64, 1, 8, 64, 2, 1>;
+using T4s = TileCfg<32, 48, 2, 4, 64, 4, 4>;
+using T4 = TileCfg<64, 48, 2, 4, 64, 2, 4>;
+using T4p = TileCfg<64, 64, 2, 4, 64, 3, 2>;
+using T2s = TileCfg<64, 48, 2, 2, 64, 2, 2>;
+using T2sp = TileCfg<64, 64, 2, 2, 64, 2, 2>;
+using T2 = TileCfg<64, 48, 4, 2, 64, 4, 4>;
+using T1s = TileCfg<32, 48, 4, 1, 64, 4, 4>;
+using T1 = TileCfg<64, 48, 4, 1, 64, 2, 4>;
+using T1b = TileCfg<128, 48, 4, 1, 64, 2, 4>;
 
-// Time model of a launch, in microseconds, from launches of 0.7 to 116
-// GFLOP on 256 CUs (within ~15 % of each): 2 + q (e + c b), q tiles per CU
-// (rounded up) of b = K / 32 / KG blocks per wave group each; a lone tile
-// of a configuration that shares a CU runs slower than one of two (c1).
+// Time model of a launch, in microseconds, from launches of every tile over
+// 32 to 2048 tokens, K 1536 to 9216, N 3072 to 18432 on 256 CUs (most within
+// 10 %): a CU runs q tiles (rounded up), `occ` at a time; each adds e + c b
+// to a busy CU, b = K / 32 / KG blocks per range, and what is left at the end
+// takes e1 + c1 b at least, a tile's time alone.
 struct TileCost {
-    double e, c, c1;
+    int occ;
+    double e, c, e1, c1;
 };
 template <class C>
 constexpr TileCost tile_cost() {
-    if (C::KG == 8) return C::BM == 32 ? TileCost{0.8, 0.40, 0.40} : TileCost{2.2, 0.56, 0.56};
-    if (C::KG == 4) return C::BM == 32 ? TileCost{1.9, 0.34, 0.34} : TileCost{2.8, 0.48, 0.48};
-    if (C::KG == 2) return C::BN == 192 ? TileCost{3.0, 0.38, 0.38} : TileCost{1.5, 0.23, 0.26};
-    if (C::BM == 32) return TileCost{0.8, 0.14, 0.20};
-    return C::BM == 64 ? TileCost{0.6, 0.19, 0.24} : TileCost{1.5, 0.335, 0.35};
+    constexpr double wide = C::WN / 48.0; // 64-column waves, by their columns
+    if (C::KG == 8) return C::BM == 32 ? TileCost{1, 1.2, 0.34 * wide, 2.0, 0.34 * wide} : TileCost{1, 2.5, 0.50 * wide, 2.5, 0.50 * wide};
+    if (C::KG == 4) return C::BM == 32 ? TileCost{1, 2.9, 0.25 * wide, 2.9, 0.25 * wide} : TileCost{1, 2.5, 0.41 * wide, 2.5, 0.41 * wide};
+    if (C::KG == 2)
+        return C::NWN == 4 ? TileCost{1, 4.0, 0.375, 4.0, 0.375}
+                           : TileCost{C::WN == 48 ? 3 : 2, 1.0, 0.195 * wide, 0.9, 0.31 * wide};
+    if (C::BM == 32) return TileCost{3, 0.9, 0.115, 1.1, 0.207};
+    return C::BM == 64 ? TileCost{3, 0.9, 0.18, 3.4, 0.25} : TileCost{2, 1.0, 0.305, 4.7, 0.365};
 }
 template <class C>
 double tile_us(int M, int K, int N, int num_cus) {
     const TileCost t = tile_cost<C>();
     const int64_t tiles = (int64_t)((M + C::BM - 1) / C::BM) * ((N + C::BN - 1) / C::BN);
-    const double q = (double)((tiles + num_cus - 1) / num_cus), b = (double)(K / 32) / C::KG;
-    return 2.0 + q * (t.e + (q > 1 ? t.c : t.c1) * b);
+    const int64_t q = (tiles + num_cus - 1) / num_cus, rest = q % t.occ;
+    const double b = (double)(K / 32) / C::KG, add = t.e + t.c * b, alone = t.e1 + t.c1 * b;
+    return 3.3 + (double)(q - rest) * add + (rest ? std::max(alone, (double)rest * add) : 0.0);
 }
 
 template <class C, int EPI>
@@ -77,18 +83,35 @@ hipError_t launch_tile(const void *packed, const uint8_t *w, int K, int N, int M
 
 } // namespace
 
-int gemm_kranges(int M, int K, int N, int num_cus) {
-    if (num_cus <= 0) num_cus = 256;
-    const int64_t mt = (M + 63) / 64;
-    auto tiles = [&](int bn) { return mt * ((N + bn - 1) / bn); };
-    int kg = 1;
-    if (4 * tiles(192) < 5 * (int64_t)num_cus) kg = tiles(48) <= num_cus ? 8 : tiles(96) <= num_cus ? 4 : 2;
-    while (kg > 1 && kg * 384 > K) kg /= 2;
-    return kg;
+double tile_gemm_us(int M, int K, int N, int num_cus, int kranges) {
+    const int cus = num_cus > 0 ? num_cus : 256;
+    auto us = [&](auto a, auto b) { return std::min(tile_us<decltype(a)>(M, K, N, cus), tile_us<decltype(b)>(M, K, N, cus)); };
+    switch (kranges) {
+    case 8: return us(T8s{}, T8{});
+    case 4: return us(T4s{}, T4{});
+    case 2: return us(T2s{}, T2{});
+    default: return std::min(us(T1s{}, T1{}), tile_us<T1b>(M, K, N, cus));
+    }
 }
 
-double tile_gemm_us(int M, int K, int N, int num_cus) {
-    return std::min({tile_us<T1s>(M, K, N, num_cus), tile_us<T1>(M, K, N, num_cus), tile_us<T1b>(M, K, N, num_cus)});
+// The fewest microseconds by the models of the tiles and, for one range, of
+// the persistent kernels; a range has at least 384 of K.  One range from 1.25
+// tiles of 64 x 192 a CU on: there a row's bits do not depend on how many rows
+// come with it, and a second range saves little (M=1500 K=3072 N=3072: 39 and
+// 37 us; below, M=300 N=9216: 32 and 25).
+int gemm_kranges(int M, int K, int N, int num_cus) {
+    int best = 1;
+    double best_us = std::min(tile_gemm_us(M, K, N, num_cus, 1), persistent_gemm_us(M, K, N, num_cus));
+    const int64_t tiles = (int64_t)((M + 63) / 64) * ((N + 191) / 192);
+    if (4 * tiles >= 5 * (int64_t)(num_cus > 0 ? num_cus : 256)) return 1;
+    for (int kg = 2; kg <= 8 && kg * 384 <= K; kg *= 2) {
+        const double us = tile_gemm_us(M, K, N, num_cus, kg);
+        if (us < best_us) {
+            best_us = us;
+            best = kg;
+        }
+    }
+    return best;
 }
 
 template <int EPI>

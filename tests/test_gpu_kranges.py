@@ -26,6 +26,8 @@ SHAPES = [  # (m, k, n), ranges on 256 CUs
     (31, 1920, 18433), (129, 2688, 9000), (512, 1536, 3072),                                                # 4
     (63, 768, 577), (200, 1152, 640), (1024, 1536, 3072),                                                   # 2
     (19, 384, 1), (63, 384, 1500), (300, 3072, 9216), (130, 768, 30000), (1000, 1152, 9217),                # 1
+    # weight groups of 2 and 4 pairs cut off by a range's end, every tile
+    (33, 3456, 300), (500, 2688, 3071), (777, 1920, 3000), (1024, 8064, 3072), (400, 384, 9217), (1100, 1152, 9000),
 ]
 
 
