@@ -1915,19 +1915,13 @@ __global__ __launch_bounds__((Gemm16Cfg<BM, BN>::NT), 2) void b1_gemm16_kernel(c
         // 12-byte pair held in d
         auto expand = [&](int j, int nt, u32x4 &bo) {
             const uint32_t *dd = d[nt];
-            uint32_t s2, wg;
-            if ((j & 1) == 0) {
-                s2 = dup_lo16(dd[0]);
-                // the sign word of block j, shifted right by 4g (bits above
-                // 27 are not those of the plain shift; only bits t and
-                // 16 + t, t < 4, reach the mask)
-                wg = __builtin_amdgcn_alignbit(dd[1], dd[0], 16 + 4 * g);
-            } else {
-                s2 = dup_hi16(dd[1]);
-                wg = dd[2] >> (4 * g);
-            }
-#pragma unroll
-            for (int t = 0; t < 4; ++t) bo[t] = wpair(wg, 15 - t, s2);
+            // the sign word of block j, shifted so that the lane's last pair,
+            // 4g + 3, is at the sign bits (bits of no pair of the lane do not
+            // reach the mask)
+            if ((j & 1) == 0)
+                bo = wpair4(__builtin_amdgcn_alignbit(dd[1], dd[0], 4 + 4 * g), dup_lo16(dd[0]));
+            else
+                bo = wpair4(dd[2] << (12 - 4 * g), dup_hi16(dd[1]));
         };
 #pragma unroll
         for (int nt = 0; nt < C::NTL; ++nt) expand(0, nt, bw[0][nt]);
