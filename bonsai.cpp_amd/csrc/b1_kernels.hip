@@ -2625,16 +2625,19 @@ __global__ __launch_bounds__(kGvWaves * 64) void b1_gemv_kernel(LinearArgs p, in
 //    two >= M).  S <= 8: one 1 KB DMA per slot, the token's 12 blocks as
 //    they lie in its row; S = 16: each 1 KB DMA carries one fragment in
 //    fragment order (g3_issue_act).  Tokens past M and slots past S zero.
-//  * Activations, fp32 (!PACKED): lane (g, tok) takes the 8 elements of its
-//    fragment slot (S = 8: from the slot slices DMAs staged in LDS,
-//    g3_issue_act_f32; S = 16: straight from the fp32 rows) and converts
-//    them to fp16 pairs (round to nearest even) in registers; a lane that
+//  * Activations, fp32 (!PACKED): converted to fp16 pairs (round to nearest
+//    even) in registers, S = 8 from the slot slices DMAs staged in LDS
+//    (g3_issue_act_f32), lane (g, tok) the 8 elements of its fragment slot,
+//    S = 16 as 4 lanes read 64 bytes of a row, then through LDS into
+//    fragments; a lane that
 //    met an |a| >= 65520 (beyond the fp16 range) flags its token, and after
 //    the reduction the work-group computes its rows of flagged tokens again
 //    in the reference's scalar arithmetic (EXACT mode's bits), correcting
 //    the non-finite count.  (Loading the fragment slots straight from the
 //    rows touches a separate 64-byte line per lane; staging the slices
-//    takes 11.1 -> 10.1 us at M=8 K=3072 N=18432.)
+//    takes 11.1 -> 10.1 us at M=8 K=3072 N=18432, the rows 64 bytes at a
+//    time 8.6 -> 6.9 us at M=12 N=9216, 12.4 -> 9.2 at M=16 N=18432 and
+//    18.9 -> 10.2 at M=12 K=9216 N=3072.)
 //  * Order of the loads: activations first, then the weight row groups, so
 //    that vmcnt (which retires in issue order) tells when each has landed.
 // One pass covers 96 blocks (K 3072, 12 per wave); longer K runs more
@@ -2909,17 +2912,17 @@ __global__ __launch_bounds__(kGvWaves * 64) void b1_gemv3_kernel(LinearArgs p, i
                 (int)(((uint32_t)(p.M - 1) * (uint32_t)p.lda + (uint32_t)p.K) * 4u), kBufferFlags);
             g3_issue_act_f32(frs, abuf, lane, wb0, nb, p.M, p.lda);
         } else {
-            // lane (g, col): elements 32 blk + 4 t .. +3 and 16 later of token
-            // col, blk = wb0 + 4 q + g, for fragment (q, t)
+            // lane (token, quad) = (lane / 4, lane % 4): elements 4 quad .. +3
+            // and 16 later of every block of the slice, so that 4 lanes read
+            // 64 consecutive bytes
 #pragma unroll
-            for (int f = 0; f < kGvBPW; ++f) {
-                const int blk = wb0 + 4 * (f >> 2) + g;
-                if (col < p.M && blk < nb) {
-                    const float *src = p.act + (size_t)col * p.lda + (size_t)blk * 32 + 4 * (f & 3);
-                    xa[f][0] = *reinterpret_cast<const floatx4 *>(src);
-                    xa[f][1] = *reinterpret_cast<const floatx4 *>(src + 16);
+            for (int b = 0; b < kGvBPW; ++b) {
+                if ((lane >> 2) < p.M && wb0 + b < nb) {
+                    const float *src = p.act + (size_t)(lane >> 2) * p.lda + (size_t)(wb0 + b) * 32 + 4 * (lane & 3);
+                    xa[b][0] = *reinterpret_cast<const floatx4 *>(src);
+                    xa[b][1] = *reinterpret_cast<const floatx4 *>(src + 16);
                 } else {
-                    xa[f][0] = xa[f][1] = floatx4{0.f, 0.f, 0.f, 0.f};
+                    xa[b][0] = xa[b][1] = floatx4{0.f, 0.f, 0.f, 0.f};
                 }
             }
         }
@@ -2952,13 +2955,26 @@ __global__ __launch_bounds__(kGvWaves * 64) void b1_gemv3_kernel(LinearArgs p, i
                 }
             }
         } else {
+            // through LDS into fragments: fragment f = 4 (b / 4) + quad at
+            // 1024 f, lane (g = b % 4, token) of it at g, token ^ 4 quad, which
+            // spreads the writes of 4 tokens' quads over the banks (written and
+            // read by this wave only: its LDS operations complete in order)
 #pragma unroll
-            for (int f = 0; f < kGvBPW; ++f)
+            for (int b = 0; b < kGvBPW; ++b) {
+                u32x4 v;
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    amax = absmax3(amax, xa[f][0][j], xa[f][1][j]);
-                    af[f >> 2][f & 3][j] = pack_f16(xa[f][0][j], xa[f][1][j]);
+                    amax = absmax3(amax, xa[b][0][j], xa[b][1][j]);
+                    v[j] = pack_f16(xa[b][0][j], xa[b][1][j]);
                 }
+                const int quad = lane & 3;
+                *reinterpret_cast<u32x4 *>(abuf + (4 * (b >> 2) + quad) * 1024 +
+                                           ((b & 3) * 16 + ((lane >> 2) ^ (4 * quad))) * 16) = v;
+            }
+#pragma unroll
+            for (int f = 0; f < kGvBPW; ++f)
+                af[f >> 2][f & 3] =
+                    *reinterpret_cast<const u32x4 *>(abuf + f * 1024 + (g * 16 + (col ^ (4 * (f & 3)))) * 16);
         }
         // 4. row group by row group, as this wave's own DMAs land
         g3_decode<0>(wbuf, nrg, wave, lane, af, acc);
@@ -2976,9 +2992,17 @@ __global__ __launch_bounds__(kGvWaves * 64) void b1_gemv3_kernel(LinearArgs p, i
         if (r < nrg) red[(wave * kGvMaxRG + r) * 64 + lane] = acc[r];
     uint32_t *flags = reinterpret_cast<uint32_t *>(gsm + kGvWaves * kGvMaxRG * 64 * 16);
     if constexpr (!PACKED) {
+        // the token whose elements a lane converted: lane % 16 (S <= 8), or
+        // lane / 4
         const uint64_t bal = __builtin_amdgcn_ballot_w64(amax >= kF16Overflow);
-        const uint32_t toks = (uint32_t)((bal | (bal >> 16) | (bal >> 32) | (bal >> 48)) & 0xFFFFu) &
-                              (p.M >= 16 ? 0xFFFFu : (1u << p.M) - 1u);
+        uint32_t toks = 0;
+        if constexpr (S <= 8) {
+            toks = (uint32_t)((bal | (bal >> 16) | (bal >> 32) | (bal >> 48)) & 0xFFFFu);
+        } else {
+#pragma unroll
+            for (int t = 0; t < 16; ++t) toks |= (uint32_t)(((bal >> (4 * t)) & 15u) != 0) << t;
+        }
+        toks &= p.M >= 16 ? 0xFFFFu : (1u << p.M) - 1u;
         if (lane == 0) flags[wave] = toks;
     }
     __syncthreads();
