@@ -178,9 +178,11 @@ def load():
 
 
 def _stream_handle(stream):
+    if stream is not None:
+        return stream.cuda_stream
+    # the current stream's raw handle without a Stream object
     import torch
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return ctypes.c_void_p(s.cuda_stream)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def linear_raw(act_ptr: int, lda: int, w_ptr: int, in_dim: int, out_dim: int, batch: int,
