@@ -56,8 +56,7 @@ constexpr int kExTN = 256; // output columns per work-group (one per thread)
 // instruction per SIMD (66 us at M=256 K=3072 N=3072), so the rest is kept
 // off the VALU.  The activations are the same in all lanes: they come by
 // scalar loads, KS elements of the TM rows a step, one step ahead, and enter
-// the FMA as its SGPR operand (as LDS broadcasts the reads were the bound:
-// 16 bytes a lane for 4 FMAs).  The signs are fp16 +-1.0 pairs (elements d
+// the FMA as its SGPR operand, with no LDS read and no barrier.  The signs are fp16 +-1.0 pairs (elements d
 // and d + 16), a shift and a bit op for two, read as halves by
 // v_fma_mix_f32, which converts them exactly and runs at the FMA's rate.
 // The packed weights arrive 24 bytes (4 blocks) at a time, one ahead.  Each
@@ -166,6 +165,74 @@ __global__ __launch_bounds__(kExTN) void b1_exact_kernel(LinearArgs p) {
         advance(128);
     }
     asm volatile("" ::"v"(warm));
+    if (n >= p.N) return;
+    int bad = 0;
+#pragma unroll
+    for (int r = 0; r < TM; ++r) {
+        if (m0 + r < p.M) {
+            bad += !__builtin_isfinite(sum[r]);
+            p.out[(size_t)(m0 + r) * p.ldo + n] = sum[r];
+        }
+    }
+    count_nonfinite(p.nonfinite, bad);
+}
+
+// EXACT mode for large grids: 8 or 16 rows a work-group share a block's fp32
+// signs (a shift and a bit op each), the rows' K chunk staged in LDS and read
+// as broadcasts: 1 + 2 / TM vector operations a multiply-accumulate, where
+// b1_exact_kernel's 4 rows, all its scalar registers hold, make 1.36.
+constexpr int kExKC = 256; // K staged in LDS per pass
+template <int TM>
+__global__ __launch_bounds__(kExTN) void b1_exact_lds_kernel(LinearArgs p) {
+#pragma clang fp contract(off)
+    __shared__ __attribute__((aligned(16))) float As[TM][kExKC];
+    const int n = blockIdx.x * kExTN + threadIdx.x;
+    const int m0 = blockIdx.y * TM;
+    const int nb = p.K / 32;
+    const int nrow = n < p.N ? n : p.N - 1;
+    const uint16_t *wr = reinterpret_cast<const uint16_t *>(p.w + (size_t)nrow * nb * 6);
+    float sum[TM];
+#pragma unroll
+    for (int r = 0; r < TM; ++r) sum[r] = 0.0f;
+
+    for (int kc = 0; kc < p.K; kc += kExKC) {
+        const int klen = min(kExKC, p.K - kc);
+        __syncthreads();
+        for (int i = threadIdx.x; i < TM * kExKC; i += kExTN) {
+            const int r = i / kExKC, c = i - r * kExKC;
+            As[r][c] = (m0 + r < p.M && c < klen)
+                           ? p.act[(size_t)(m0 + r) * p.lda + kc + c]
+                           : 0.0f;
+        }
+        __syncthreads();
+        const int nbk = klen / 32;
+        for (int b = 0; b < nbk; ++b) {
+            const uint16_t *blk = wr + (size_t)(kc / 32 + b) * 3;
+            const float scale = (float)__builtin_bit_cast(_Float16, blk[0]);
+            const uint32_t bits = (uint32_t)blk[1] | ((uint32_t)blk[2] << 16);
+            float bs[TM];
+#pragma unroll
+            for (int r = 0; r < TM; ++r) bs[r] = 0.0f;
+#pragma unroll
+            for (int i4 = 0; i4 < 8; ++i4) {
+                // +1.0 for a set bit, -1.0 for a clear one
+                float sg[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int i = 4 * i4 + j;
+                    sg[j] = __builtin_bit_cast(float, ((bits << (31 - i)) & 0x80000000u) ^ 0xBF800000u);
+                }
+#pragma unroll
+                for (int r = 0; r < TM; ++r) {
+                    const floatx4 a = *reinterpret_cast<const floatx4 *>(&As[r][b * 32 + 4 * i4]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) bs[r] = __builtin_fmaf(a[j], sg[j], bs[r]);
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < TM; ++r) sum[r] = sum[r] + scale * bs[r];
+        }
+    }
     if (n >= p.N) return;
     int bad = 0;
 #pragma unroll
@@ -3399,6 +3466,17 @@ hipError_t launch_exact(const LinearArgs &a, int num_cus, hipStream_t s) {
         const double busy = (double)((wgs + cus - 1) / cus) * add;
         return busy > alone ? busy : alone;
     };
+    // 16 or 8 rows through LDS while that leaves at least 4 work-groups (16
+    // waves) a CU (M=1024 K=3072 N=4768: 565 us, with 4 rows 611; M=4096
+    // N=12288 4.96 ms, 5.99; M=256 N=3072, below, 151 with 4 rows, 107)
+    if (a.M > 8 && cols * ((a.M + 15) / 16) >= 4 * cus) {
+        hipLaunchKernelGGL((b1_exact_lds_kernel<16>), dim3((unsigned)cols, (unsigned)((a.M + 15) / 16)), dim3(kExTN), 0, s, a);
+        return hipGetLastError();
+    }
+    if (a.M > 4 && cols * ((a.M + 7) / 8) >= 4 * cus) {
+        hipLaunchKernelGGL((b1_exact_lds_kernel<8>), dim3((unsigned)cols, (unsigned)((a.M + 7) / 8)), dim3(kExTN), 0, s, a);
+        return hipGetLastError();
+    }
     const double us1 = us(1, 11.8, 15.0), us2 = us(2, 17.4, 22.0), us4 = us(4, 31.5, 38.0);
     auto go = [&](auto kernel, int tm) {
         const dim3 grid((unsigned)cols, (unsigned)((a.M + (int64_t)tm - 1) / tm));

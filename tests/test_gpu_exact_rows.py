@@ -1,5 +1,5 @@
 """EXACT mode's kernel (b1_exact_kernel: 1, 2 or 4 rows a work-group, scalar
-activation loads, weights 4 blocks at a time) against the oracle's scalar
+activation loads, weights 4 blocks at a time; b1_exact_lds_kernel: 8 or 16) against the oracle's scalar
 order, bit for bit.
 
 Shapes: the three row counts on 256 CUs, row remainders, widths around the
@@ -19,6 +19,7 @@ SHAPES = [  # (m, k, n)
     (1, 32, 1), (1, 3072, 257), (3, 96, 255), (5, 128, 513), (7, 160, 300),      # 1 row
     (65, 224, 1000), (301, 64, 600), (130, 256, 769), (103, 416, 1024),          # 2 rows
     (201, 288, 3000), (258, 1056, 1003), (1023, 192, 1500), (130, 128, 5000),    # 4 rows
+    (601, 96, 3600), (1030, 288, 4090),                                          # 8 and 16 (through LDS)
 ]
 
 
