@@ -244,13 +244,12 @@ static b1::LinearArgs linear_args(const float *act, int64_t lda, const void *w, 
     return a;
 }
 
-// The workspace size the queries report for these arguments: the FAST
-// GEMM's range-safe packing and gemm_partial_bytes; none for the small-M
-// kernel and EXACT mode.
-static size_t linear_need(const b1::LinearArgs &a, int mode, int num_cus) {
+// The workspace of the kernel these arguments run: the FAST GEMM's
+// range-safe packing; none for the small-M kernel and EXACT mode.
+static size_t linear_need(const b1::LinearArgs &a, int mode) {
     if (mode == BONSAI_B1_MODE_EXACT || mode == BONSAI_B1_MODE_GEMV) return 0;
     if (mode != BONSAI_B1_MODE_GEMM && b1::gemv_supported(a)) return 0;
-    return b1::gemm_supported(a) ? b1::gemm_workspace_bytes_total(a, num_cus) : 0;
+    return b1::gemm_supported(a) ? b1::gemm_workspace_bytes(a) : 0;
 }
 
 // Shared body of the two linear entry points.  ws_mode: 0 = library-owned
@@ -327,9 +326,7 @@ size_t bonsai_b1_workspace_bytes(int batch, int in_dim, int out_dim, int mode) {
     a.w = reinterpret_cast<const uint8_t *>(uintptr_t(256));
     // the small-M kernel converts the activations itself
     if (mode == BONSAI_B1_MODE_GEMV || (mode != BONSAI_B1_MODE_GEMM && batch <= b1::kGemvMaxM)) return 0;
-    // the range-safe packing, then gemm_partial_bytes (0 without a device)
-    const DeviceInfo *dev = current_device(nullptr);
-    return b1::gemm_workspace_bytes_total(a, dev ? dev->num_cus : 0);
+    return b1::gemm_workspace_bytes(a); // the range-safe packing
 }
 
 int bonsai_b1_linear_f32_ws(const float *act, int64_t lda, const void *w,
@@ -354,7 +351,7 @@ int bonsai_b1_linear_f32_noalloc(const float *act, int64_t lda, const void *w, i
     // what the kernel this call runs would use (an unaligned call runs EXACT
     // mode and needs none)
     const b1::LinearArgs a = linear_args(act, lda, w, in_dim, out_dim, batch, out, ldo, nonfinite);
-    if (linear_need(a, mode, dev->num_cus) > BONSAI_B1_NOALLOC_SCRATCH_BYTES) return BONSAI_B1_ERR_SCRATCH;
+    if (linear_need(a, mode) > BONSAI_B1_NOALLOC_SCRATCH_BYTES) return BONSAI_B1_ERR_SCRATCH;
     void *ws = device_scratch(dev);
     if (!ws) return BONSAI_B1_ERR_HIP;
     return linear_impl(act, lda, w, in_dim, out_dim, batch, out, ldo, mode, nonfinite, 1, ws,
@@ -490,7 +487,7 @@ size_t bonsai_b1_linear_packed_workspace_bytes(int batch, int in_dim, int out_di
     if (batch <= 0 || in_dim <= 0 || out_dim <= 0 || !b1::gemm_packed_ok(batch, in_dim, out_dim)) return 0;
     if (b1::gemv_packed_ok(batch, in_dim, out_dim)) return 0;
     const DeviceInfo *dev = current_device(nullptr);
-    return b1::gemm_partial_bytes(batch, in_dim, out_dim, out_dim, dev ? dev->num_cus : 0);
+    return b1::gemm_partial_bytes(batch, in_dim, out_dim, dev ? dev->num_cus : 0);
 }
 
 // Shared body of the packed entry points (ws: checked, not used).
@@ -926,21 +923,18 @@ static int gemv_span(int n_ops, int mode, OpAt at, int i, b1::GemvGroupOp *ops, 
     return i + n - 1;
 }
 
-// Workspace areas of a batch, laid out [pack][split][y], each 256-byte
-// aligned: the largest range-safe packing among its packed GEMMs and
-// grouped small-M runs of more than kGemvGroupF32MaxM tokens, the largest
-// gemm_partial_bytes among its plain packed GEMMs (fused runs included; part
-// of the reported size only), and the largest fp32 linear output among its
-// ops whose epilogue runs as a separate pass (the other paths).
+// Workspace areas of a batch, laid out [pack][y], each 256-byte aligned: the
+// largest range-safe packing among its packed GEMMs and grouped small-M runs
+// of more than kGemvGroupF32MaxM tokens, and the largest fp32 linear output
+// among its ops whose epilogue runs as a separate pass (the other paths).
 struct BatchAreas {
-    size_t pack = 0, split = 0, y = 0;
-    size_t split_off() const { return round256(pack); }
-    size_t y_off() const { return split_off() + round256(split); }
-    size_t need() const { return y ? y_off() + y : split ? split_off() + split : pack; }
+    size_t pack = 0, y = 0;
+    size_t y_off() const { return round256(pack); }
+    size_t need() const { return y ? y_off() + y : pack; }
 };
 
 template <class OpAt>
-static BatchAreas batch_areas(int n_ops, int mode, int num_cus, OpAt at, bool pack_groups = true) {
+static BatchAreas batch_areas(int n_ops, int mode, OpAt at, bool pack_groups = true) {
     BatchAreas r;
     for (int i = 0; i < n_ops; ++i) {
         const BatchOp b = at(i);
@@ -956,14 +950,8 @@ static BatchAreas batch_areas(int n_ops, int mode, int num_cus, OpAt at, bool pa
                 continue;
             }
         }
-        if (path == BatchPath::Packed) r.pack = std::max(r.pack, b1::pack_area_bytes(a.M, a.K));
         if (path == BatchPath::Packed) {
-            if (epi_kind(b.epi) == BONSAI_B1_EPI_NONE) {
-                int n_sum;
-                const int last = fuse_span(n_ops, mode, num_cus, at, i, &n_sum);
-                r.split = std::max(r.split, b1::gemm_partial_bytes(a.M, a.K, a.N, n_sum, num_cus));
-                i = last;
-            }
+            r.pack = std::max(r.pack, b1::pack_area_bytes(a.M, a.K));
         } else if (epi_kind(b.epi) != BONSAI_B1_EPI_NONE) {
             r.y = std::max(r.y, (size_t)a.M * (size_t)a.N * sizeof(float));
         }
@@ -973,8 +961,7 @@ static BatchAreas batch_areas(int n_ops, int mode, int num_cus, OpAt at, bool pa
 
 template <class OpAt>
 static size_t batch_need(int n_ops, int mode, OpAt at) {
-    const DeviceInfo *dev = current_device(nullptr);
-    return batch_areas(n_ops, mode, dev ? dev->num_cus : 0, at).need();
+    return batch_areas(n_ops, mode, at).need();
 }
 
 template <class OpAt>
@@ -995,20 +982,19 @@ static int batch_run(int n_ops, int mode, int32_t *nonfinite, void *workspace, s
     }
     DeviceInfo *dev = current_device(nullptr);
     if (!dev) return BONSAI_B1_ERR_DEVICE;
-    BatchAreas areas = batch_areas(n_ops, mode, dev->num_cus, at);
+    BatchAreas areas = batch_areas(n_ops, mode, at);
     WsLease lease;
     bool pack_groups = true;
     if (areas.need() > 0) {
         if (!workspace) {
-            areas.split = 0; // no kernel uses that area
-            if (areas.need() > 0) lease.acquire(dev, stream, areas.need());
+            lease.acquire(dev, stream, areas.need());
             workspace = lease.ptr();
             workspace_bytes = workspace ? areas.need() : 0;
             if (!workspace) {
                 // No library workspace to be had (a capture with no large
                 // enough buffer): grouped small-M runs that would read a
                 // packing run their ops one by one instead, which needs none.
-                const BatchAreas alone = batch_areas(n_ops, mode, dev->num_cus, at, false);
+                const BatchAreas alone = batch_areas(n_ops, mode, at, false);
                 if (alone.need() == 0) {
                     areas = alone;
                     pack_groups = false;
@@ -1017,8 +1003,6 @@ static int batch_run(int n_ops, int mode, int32_t *nonfinite, void *workspace, s
         }
     }
     if (areas.need() > 0) {
-        // (a workspace need not hold that area)
-        if (workspace && workspace_bytes < areas.need()) areas.split = 0;
         if (!workspace || workspace_bytes < areas.need() || (reinterpret_cast<uintptr_t>(workspace) & 15u))
             return BONSAI_B1_ERR_ARG;
         if (!lease.ptr()) {

@@ -50,14 +50,10 @@ hipError_t launch_exact(const LinearArgs &a, int num_cus, hipStream_t s);
 // staging each tile and computes rows beyond the fp16 range exactly itself.
 bool gemm_supported(const LinearArgs &a);
 size_t gemm_workspace_bytes(const LinearArgs &a);
-// The size callers are told: the packing and the area gemm_partial_bytes
-// describes (which no kernel uses).
-size_t gemm_workspace_bytes_total(const LinearArgs &a, int num_cus);
 hipError_t launch_gemm(const LinearArgs &a, int num_cus, void *workspace, size_t ws_bytes, hipStream_t s);
 
-// Bytes the size queries report beyond the packing (n_sum: the width of a
-// run of linears issued as one).
-size_t gemm_partial_bytes(int M, int K, int N, int n_sum, int num_cus);
+// Bytes bonsai_b1_linear_packed_workspace_bytes reports (no kernel uses them).
+size_t gemm_partial_bytes(int M, int K, int N, int num_cus);
 
 // The number of contiguous K ranges a packed GEMM sums separately and then
 // adds in order (1, 2, 4 or 8), a function of the shape and CU count only,

@@ -3589,13 +3589,13 @@ hipError_t launch_pack(const float *act, int64_t lda, int M, int K, void *packed
     return hipGetLastError();
 }
 
-// What the size queries report beyond the packing: S fp32 partial products
-// of M x N (rows rounded up to 4 columns) for shapes whose 128 x 512 tiles
-// leave more than half of the CUs idle, S from a time model of that kernel
-// (10.9 us per 384-K unit of a tile, partials at ~5 TB/s, 3 us for their
-// sum).  The K ranges are now summed in LDS (b1_tile_gemm.h) and no kernel
-// uses this area; the sizes stay what callers have laid buffers out by.
-size_t gemm_partial_bytes(int M, int K, int N, int n_sum, int num_cus) {
+// What bonsai_b1_linear_packed_workspace_bytes reports: S fp32 partial
+// products of M x N (rows rounded up to 4 columns) for shapes whose 128 x 512
+// tiles leave more than half of the CUs idle, S from a time model of that
+// kernel (10.9 us per 384-K unit of a tile, partials at ~5 TB/s, 3 us for
+// their sum).  The K ranges are now summed in LDS (b1_tile_gemm.h) and no
+// kernel uses this area; that query's results stay what they were.
+size_t gemm_partial_bytes(int M, int K, int N, int num_cus) {
     if (num_cus <= 0 || !gemm_packed_ok(M, K, N) || N % 4) return 0;
     const int tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN);
     const int slots = num_cus * kWgPerCu;
@@ -3613,7 +3613,7 @@ size_t gemm_partial_bytes(int M, int K, int N, int n_sum, int num_cus) {
             best_us = us;
         }
     }
-    return best > 1 ? (size_t)best * (size_t)M * (size_t)((n_sum + 3) & ~3) * sizeof(float) : 0;
+    return best > 1 ? (size_t)best * (size_t)M * (size_t)((N + 3) & ~3) * sizeof(float) : 0;
 }
 
 // Rounds of the 128 x 512 kernel's persistent grid, in units of one round
@@ -3830,11 +3830,6 @@ hipError_t launch_gemm(const LinearArgs &a, int num_cus, void *workspace, size_t
     epi.rsc = pack_area_rsc(workspace, a.M, a.K);
     return launch_gemm_packed_epi(workspace, a.w, a.K, a.N, a.M, a.out, a.ldo, a.nonfinite, num_cus,
                                   gemm_kranges(a.M, a.K, a.N, num_cus), 0, epi, s);
-}
-
-size_t gemm_workspace_bytes_total(const LinearArgs &a, int num_cus) {
-    const size_t pack = gemm_workspace_bytes(a);
-    return pack ? pack + gemm_partial_bytes(a.M, a.K, a.N, a.N, num_cus) : 0;
 }
 
 hipError_t launch_quantize(const float *w, int64_t ldw, int K, int N, void *packed, int order, hipStream_t s) {

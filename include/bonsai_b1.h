@@ -116,7 +116,7 @@ int bonsai_b1_linear_f32(const float *act, int64_t lda, const void *w,
 
 /*
  * The GEMM kernels pack the activations to fp16 once (with the row scales
- * of the range-safe packing) into a device workspace, at most
+ * of the range-safe packing) into a device workspace of
  * bonsai_b1_workspace_bytes(batch, in_dim, out_dim, mode) bytes (0 when the
  * call needs none: EXACT, and small batches, whose kernel converts the
  * activations itself).  bonsai_b1_linear_f32 keeps library-owned workspaces

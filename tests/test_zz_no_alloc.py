@@ -135,3 +135,30 @@ def test_noalloc_under_graph_capture(torch, lib):
         torch.cuda.synchronize()
         say(f"  replay {i}: max |diff| {float((y - ref).abs().max()):.3e}")
         assert torch.equal(y, ref), f"replay {i}"
+
+
+@pytest.mark.parametrize("m,k,n", [(512, 3072, 3072), (512, 9216, 3072), (1024, 3072, 3072)])
+def test_need_is_the_packing_alone(torch, lib, m, k, n):
+    """Shapes with few output tiles, whose K the GEMM sums in ranges: no
+    partial product goes to memory, so what the calls need is the fp16
+    packing and the row scales, far below the static array.  The size queries
+    say so, the no-alloc entry runs, and a batch takes a caller's buffer that
+    holds the packing with the output right behind it."""
+    import bonsai_b1 as b1
+    from bonsai_b1 import capi, synth
+    say(f"no-alloc need ({m},{k},{n})")
+    pack = (m * k * 2 + 255) // 256 * 256 + (m * 4 + 255) // 256 * 256
+    assert capi.workspace_bytes(m, k, n, "auto") == pack
+    a = synth.device_activations(m, k, 81)
+    w = synth.device_packed_weights(n, k, 82)
+    ref = torch.full((m, n), 3.0, device="cuda")
+    got = torch.full((m, n), 5.0, device="cuda")
+    assert _call(lib, torch, "bonsai_b1_linear_f32", a, w, n, ref, "auto") == capi.OK
+    assert _call(lib, torch, "bonsai_b1_linear_f32_noalloc", a, w, n, got, "auto") == capi.OK
+    buf = torch.zeros(pack // 4 + m * n, device="cuda")
+    out = buf[pack // 4:].view(m, n)
+    ops = [(a, b1.device_weights(w, k, n), out)]
+    assert capi.linear_batch_workspace_bytes(ops) == pack
+    b1.linear_batch(ops, workspace=buf)
+    torch.cuda.synchronize()
+    assert torch.equal(got, ref) and torch.equal(out, ref)
