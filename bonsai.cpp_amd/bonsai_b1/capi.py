@@ -180,9 +180,13 @@ def load():
 def _stream_handle(stream):
     if stream is not None:
         return stream.cuda_stream
-    # the current stream's raw handle without a Stream object
+    # the current stream's raw handle without a Stream object (2 us a call
+    # less), where this torch has that call
     import torch
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is None:
+        return torch.cuda.current_stream().cuda_stream
+    return raw(torch.cuda.current_device())
 
 
 def linear_raw(act_ptr: int, lda: int, w_ptr: int, in_dim: int, out_dim: int, batch: int,

@@ -53,6 +53,23 @@ def test_new_entries_reject_before_device():
                                               None) == capi.ERR_ARG
 
 
+def test_current_stream_with_and_without_the_raw_call(monkeypatch):
+    """The entry points' default stream is torch's current one: by torch's raw
+    call where it has one, else from the Stream object."""
+    import torch
+
+    class Stream:
+        cuda_stream = 0x5150
+
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 3)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 0x1000 + device, raising=False)
+    assert capi._stream_handle(None) == 0x1003
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    assert capi._stream_handle(None) == 0x5150
+    assert capi._stream_handle(Stream) == 0x5150
+
+
 @pytest.mark.parametrize("args", [
     # (lda, in_dim, out_dim, batch, ldo, mode)
     (64, 63, 32, 1, 32, 0),      # in_dim % 32 != 0 (reference precondition)
