@@ -68,9 +68,15 @@ int gemm_kranges(int M, int K, int N, int num_cus);
 hipError_t launch_tile_gemm(const void *packed, const uint8_t *w, int K, int N, int M, float *out, int64_t ldo,
                             int32_t *nonfinite, int num_cus, int kranges, int kind, const GemmEpi &epi,
                             hipStream_t s);
-// Modelled us of the K-range tiles at a number of ranges, and of the best
-// persistent kernel.
+// The tile a K-range GEMM takes.
+struct TileShape {
+    int kranges, bm, bn;
+};
+TileShape tile_shape(int M, int K, int N, int num_cus, int kranges, bool packed_out);
+// Modelled us of the K-range tiles at a number of ranges, of the one-range
+// tile with a packed output, and of the best persistent kernel.
 double tile_gemm_us(int M, int K, int N, int num_cus, int kranges);
+double packed_tile_us(int M, int K, int N, int num_cus, bool swiglu);
 double persistent_gemm_us(int M, int K, int N, int num_cus);
 
 // The two halves of the workspace path.  Packed activations: u32 word
@@ -109,6 +115,14 @@ hipError_t launch_fixup_rows(const LinearArgs &a, hipStream_t s);
 hipError_t launch_gemm_packed_epi(const void *packed, const uint8_t *w, int K, int N, int M, float *out,
                                   int64_t ldo, int32_t *nonfinite, int num_cus, int kranges, int kind,
                                   const GemmEpi &epi, hipStream_t s);
+
+// What launch_gemm_packed_epi runs for a shape (kind, act and split of its
+// epilogue), by name: "128x512", "128x512+64" (the rows after the full rounds
+// as 64-row tiles), "144x384", "128x384", or "k<ranges> <rows>x<columns>" for
+// a K-range tile.  For the tests, which ask it whether a shape still reaches
+// the kernel that they are about; no part of the C ABI.
+extern "C" void b1_gemm_plan(int M, int K, int N, int num_cus, int kind, int act, int split, char *name,
+                             size_t size);
 
 // The epilogue (kind 1 or 2) as a separate pass over y [M][ldy] (N columns
 // of y; kind 2 writes glu_h of them).

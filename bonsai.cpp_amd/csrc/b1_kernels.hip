@@ -32,6 +32,7 @@
 // unchanged.
 #include <hip/hip_runtime.h>
 
+#include <cstdio>
 #include <mutex>
 
 #include "b1_device.h"
@@ -3616,17 +3617,23 @@ size_t gemm_partial_bytes(int M, int K, int N, int num_cus) {
     return best > 1 ? (size_t)best * (size_t)M * (size_t)((N + 3) & ~3) * sizeof(float) : 0;
 }
 
+// The whole tile rows of the 128 x 512 kernel's full rounds, where the rows
+// after them run as 64-row tiles in a second launch (launch_gemm_packed_t),
+// else 0.
+static int head_tile_rows(int M, int N, int num_cus) {
+    const int tiles_n = (N + kBN - 1) / kBN, tiles = ((M + kBM - 1) / kBM) * tiles_n;
+    const int slots = num_cus > 0 ? num_cus * kWgPerCu : tiles;
+    const int full = num_cus > 0 ? tiles / slots * slots : 0, head_rows = full / tiles_n;
+    const int tail_tiles = ((M - head_rows * kBM + kBMH - 1) / kBMH) * tiles_n;
+    return full > 0 && full < tiles && tiles_n < slots && tail_tiles <= slots ? head_rows : 0;
+}
+
 // Rounds of the 128 x 512 kernel's persistent grid, in units of one round
 // of full tiles: ceil(tiles / slots), or, where launch_gemm_packed_t runs
 // the last partial round as 64-row tiles, the full rounds plus ~0.6.
 static double gemm_rounds128(int M, int N, int num_cus) {
-    const int tiles_n = (N + kBN - 1) / kBN, tiles = ((M + kBM - 1) / kBM) * tiles_n;
-    const int slots = num_cus * kWgPerCu;
-    const int full = tiles / slots * slots, head_rows = full / tiles_n;
-    const int tail_tiles = ((M - head_rows * kBM + kBMH - 1) / kBMH) * tiles_n;
-    if (full > 0 && full < tiles && tiles_n < slots && head_rows > 0 && tail_tiles <= slots)
-        return full / slots + 0.6;
-    return (double)((tiles + slots - 1) / slots);
+    const int tiles = ((M + kBM - 1) / kBM) * ((N + kBN - 1) / kBN), slots = num_cus * kWgPerCu;
+    return head_tile_rows(M, N, num_cus) ? tiles / slots + 0.6 : (double)((tiles + slots - 1) / slots);
 }
 
 // The persistent kernel a packed GEMM takes, by rounds of the grid: ~87 us a
@@ -3658,15 +3665,34 @@ double persistent_gemm_us(int M, int K, int N, int num_cus) {
 }
 
 // The kernel a packed GEMM whose K is one range runs: the faster by the time
-// models of the persistent kernels and of the K-range tiles, the latter only
-// where it is 7 % better, the scatter of both models (M=1024 K=3072 N=18432:
-// 130.7 us as two 75 % full rounds of 128 x 384, 107 us as 768 tiles of 128 x
-// 192; M=4096 N=12288: 253 us as three full rounds, 300 us modelled for the
-// others).
-static GemmKernel gemm_kernel(int M, int K, int N, int num_cus) {
+// models of the persistent kernels and of the K-range tiles, the latter where
+// it is 7 % better (us with the persistent kernel and with K-range tiles:
+// M=1024 K=3072 N=18432 123 and 113, M=4592 N=12288 320 and 304, M=4240 N=9216
+// 222 and 225, M=4096 N=12288 261 and 270).
+//  * Packed outputs, by packed_tile_us: 2 % better (SwiGLU: M=4592 K=3072
+//    N=12288 310 and 320, M=3744 K=768 N=19456 126 and 147, M=1024 K=3072
+//    N=18432 126 and 118).  Over 713 shapes of 300 to 4608 tokens K-range tiles
+//    are then taken where the persistent kernel is over 3 % faster 8 times, by
+//    up to 6 %; with the plain model and 7 %, 68 times, by up to 26 %.
+//  * Gate and residual over 512 MB of residual and output, twice the
+//    memory-side cache: the persistent kernel, whose tiles read and write
+//    longer rows (M=2836 K=1152 N=24640 234 and 266, M=3968 K=1536 N=26304 391
+//    and 438; none of 15 such shapes was over 3 % faster with K-range tiles).
+static GemmKernel gemm_kernel(int M, int K, int N, int num_cus, int kind, bool swiglu) {
     double rounds;
-    const GemmKernel kind = persistent_kernel(M, N, num_cus, &rounds);
-    return tile_gemm_us(M, K, N, num_cus, 1) < 0.93 * persistent_gemm_us(M, K, N, num_cus) ? GemmKernel::KRange : kind;
+    const GemmKernel persistent = persistent_kernel(M, N, num_cus, &rounds);
+    if (kind == 1 && (int64_t)M * N * 8 > (int64_t(512) << 20)) return persistent;
+    const double us = kind == 3 ? packed_tile_us(M, K, N, num_cus, swiglu) : tile_gemm_us(M, K, N, num_cus, 1);
+    const double limit = (kind == 3 ? 0.98 : 0.93) * persistent_gemm_us(M, K, N, num_cus);
+    return us < limit ? GemmKernel::KRange : persistent;
+}
+
+// (a packed SwiGLU output on 16x16 tiles needs the split point on a tile
+// boundary, every tile wholly fp32 or wholly SwiGLU pairs; otherwise it runs
+// the 128 x 512 kernel)
+static GemmKernel gemm_kernel_epi(int M, int K, int N, int num_cus, int kind, int act, int split) {
+    const GemmKernel t = gemm_kernel(M, K, N, num_cus, kind, act == 2);
+    return t != GemmKernel::KRange && kind == 3 && act == 2 && split % 384 != 0 ? GemmKernel::Tile128x512 : t;
 }
 
 template <int BM, int BN, int EPI>
@@ -3700,16 +3726,14 @@ template <int EPI>
 static hipError_t launch_gemm_packed_t(const void *packed, const uint8_t *w, int K, int N, int M, float *out,
                                        int64_t ldo, int32_t *nonfinite, int num_cus, const GemmEpi &epi,
                                        hipStream_t s) {
-    // (a packed SwiGLU output on 16x16 tiles needs the split point on a
-    // tile boundary, every tile wholly fp32 or wholly SwiGLU pairs; otherwise
-    // it runs the 128 x 512 kernel)
-    const GemmKernel t = gemm_kernel(M, K, N, num_cus);
-    if (t == GemmKernel::KRange) return launch_tile_gemm(packed, w, K, N, M, out, ldo, nonfinite, num_cus, 1, EPI, epi, s);
-    if (!(EPI == 3 && epi.act == 2 && epi.split % 384 != 0)) {
-        if (t == GemmKernel::Tile144x384)
-            return launch_gemm16_t<144, 384, EPI>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
-        if (t == GemmKernel::Tile128x384)
-            return launch_gemm16_t<128, 384, EPI>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
+    switch (gemm_kernel_epi(M, K, N, num_cus, EPI, epi.act, epi.split)) {
+    case GemmKernel::KRange:
+        return launch_tile_gemm(packed, w, K, N, M, out, ldo, nonfinite, num_cus, 1, EPI, epi, s);
+    case GemmKernel::Tile144x384:
+        return launch_gemm16_t<144, 384, EPI>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
+    case GemmKernel::Tile128x384:
+        return launch_gemm16_t<128, 384, EPI>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
+    case GemmKernel::Tile128x512: break;
     }
     auto kernel = &b1_gemm_kernel<kBM, kBN, kWN, kStages, EPI>;
     static std::once_flag attr_once;
@@ -3741,11 +3765,7 @@ static hipError_t launch_gemm_packed_t(const void *packed, const uint8_t *w, int
     // at M=4096 N=9216: 504 tiles in 2 rounds, then 144 half tiles instead
     // of a third round of 72).  Every output is the same sum in the same
     // order.
-    const int tiles = tiles_m * tiles_n;
-    const int full = num_cus > 0 ? tiles / slots * slots : 0;
-    const int head_rows = full / tiles_n;                        // whole tile rows in the full rounds
-    const int tail_tiles = ((M - head_rows * kBM + kBMH - 1) / kBMH) * tiles_n;
-    if (full > 0 && full < tiles && tiles_n < slots && head_rows > 0 && tail_tiles <= slots) {
+    if (const int head_rows = head_tile_rows(M, N, num_cus)) {
         auto tail = &b1_gemm_kernel<kBMH, kBN, kWN, kStages, EPI>;
         static std::once_flag tail_once;
         static hipError_t tail_err = hipSuccess;
@@ -3787,6 +3807,22 @@ hipError_t launch_gemm_packed_epi(const void *packed, const uint8_t *w, int K, i
     case 2: return launch_gemm_packed_t<2>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
     case 3: return launch_gemm_packed_t<3>(packed, w, K, N, M, out, ldo, nonfinite, num_cus, epi, s);
     default: return hipErrorInvalidValue;
+    }
+}
+
+extern "C" void b1_gemm_plan(int M, int K, int N, int num_cus, int kind, int act, int split, char *name,
+                             size_t size) {
+    const int kranges = gemm_kranges(M, K, N, num_cus);
+    const GemmKernel t =
+        kranges > 1 ? GemmKernel::KRange : gemm_kernel_epi(M, K, N, num_cus, kind, act, split);
+    if (t == GemmKernel::KRange) {
+        const TileShape c = tile_shape(M, K, N, num_cus, kranges, kind == 3);
+        snprintf(name, size, "k%d %dx%d", c.kranges, c.bm, c.bn);
+    } else {
+        snprintf(name, size, "%s", t == GemmKernel::Tile144x384   ? "144x384"
+                                   : t == GemmKernel::Tile128x384 ? "128x384"
+                                   : head_tile_rows(M, N, num_cus) ? "128x512+64"
+                                                                   : "128x512");
     }
 }
 

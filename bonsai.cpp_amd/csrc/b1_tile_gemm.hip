@@ -33,7 +33,8 @@ using T1b = TileCfg<128, 48, 4, 1, 64, 2, 4>;
 
 // Time model of a launch, in microseconds, from launches of every tile over
 // 32 to 2048 tokens, K 1536 to 9216, N 3072 to 18432 on 256 CUs (most within
-// 10 %): a CU runs q tiles (rounded up), `occ` at a time; each adds e + c b
+// 10 %; up to 4608 tokens the 128-row tile takes up to 8 % more than modelled,
+// M=4592 N=12288 307 us for 285): a CU runs q tiles (rounded up), `occ` at a time; each adds e + c b
 // to a busy CU, b = K / 32 / KG blocks per range, and what is left at the end
 // takes e1 + c1 b at least, a tile's time alone.
 struct TileCost {
@@ -51,9 +52,11 @@ constexpr TileCost tile_cost() {
     if (C::BM == 32) return TileCost{3, 0.9, 0.115, 1.1, 0.207};
     return C::BM == 64 ? TileCost{3, 0.9, 0.18, 3.4, 0.25} : TileCost{2, 1.0, 0.305, 4.7, 0.365};
 }
+// `more`: us a tile's epilogue takes beyond a plain one's.
 template <class C>
-double tile_us(int M, int K, int N, int num_cus) {
-    const TileCost t = tile_cost<C>();
+double tile_us(int M, int K, int N, int num_cus, double more = 0.0) {
+    TileCost t = tile_cost<C>();
+    t.e += more, t.e1 += more;
     const int64_t tiles = (int64_t)((M + C::BM - 1) / C::BM) * ((N + C::BN - 1) / C::BN);
     const int64_t q = (tiles + num_cus - 1) / num_cus, rest = q % t.occ;
     const double b = (double)(K / 32) / C::KG, add = t.e + t.c * b, alone = t.e1 + t.c1 * b;
@@ -114,32 +117,60 @@ int gemm_kranges(int M, int K, int N, int num_cus) {
     return best;
 }
 
-template <int EPI>
-static hipError_t tile_gemm_t(const void *packed, const uint8_t *w, int K, int N, int M, float *out, int64_t ldo,
-                              int32_t *nonfinite, int num_cus, int kranges, const GemmEpi &epi, hipStream_t s) {
+// run(tile) with the tile a GEMM of `kranges` K ranges takes (PACKED: with the
+// packed-output epilogue, which needs whole 64-column blocks).
+template <bool PACKED, class Run>
+static auto with_tile(int M, int K, int N, int num_cus, int kranges, Run run) {
     const int cus = num_cus > 0 ? num_cus : 256;
-#define B1_TILE(C) launch_tile<C, EPI>(packed, w, K, N, M, out, ldo, nonfinite, epi, s)
 #define B1_LESS(A, B) (tile_us<A>(M, K, N, cus) < tile_us<B>(M, K, N, cus))
-    // (the packed output takes tiles of whole 64-column blocks)
-    if constexpr (EPI == 3) {
+    if constexpr (PACKED) {
         switch (kranges) {
-        case 8: return B1_LESS(T8sp, T8p) ? B1_TILE(T8sp) : B1_TILE(T8p);
-        case 4: return B1_TILE(T4p);
-        case 2: return B1_LESS(T2sp, T2) ? B1_TILE(T2sp) : B1_TILE(T2);
+        case 8: return B1_LESS(T8sp, T8p) ? run(T8sp{}) : run(T8p{});
+        case 4: return run(T4p{});
+        case 2: return B1_LESS(T2sp, T2) ? run(T2sp{}) : run(T2{});
         default: break;
         }
     } else {
         switch (kranges) {
-        case 8: return B1_LESS(T8s, T8) ? B1_TILE(T8s) : B1_TILE(T8);
-        case 4: return B1_LESS(T4s, T4) ? B1_TILE(T4s) : B1_TILE(T4);
-        case 2: return B1_LESS(T2s, T2) ? B1_TILE(T2s) : B1_TILE(T2);
+        case 8: return B1_LESS(T8s, T8) ? run(T8s{}) : run(T8{});
+        case 4: return B1_LESS(T4s, T4) ? run(T4s{}) : run(T4{});
+        case 2: return B1_LESS(T2s, T2) ? run(T2s{}) : run(T2{});
         default: break;
         }
     }
-    if (B1_LESS(T1s, T1) && B1_LESS(T1s, T1b)) return B1_TILE(T1s);
-    return B1_LESS(T1, T1b) ? B1_TILE(T1) : B1_TILE(T1b);
-#undef B1_TILE
+    if (B1_LESS(T1s, T1) && B1_LESS(T1s, T1b)) return run(T1s{});
+    return B1_LESS(T1, T1b) ? run(T1{}) : run(T1b{});
 #undef B1_LESS
+}
+
+// A packed output's epilogue (fp16 pairs, GELU) counts 1 us more than a plain
+// one's in a 64-row tile and 2 in a 128-row one, with SwiGLU 1.5 and 5, from
+// 713 launches of each over 300 to 4608 tokens: fewer work-groups a CU leave
+// more of it bare (M=1024 K=3072 N=18432, six 64-row or three 128-row tiles a
+// CU: plain 114 and 111 us, packed SwiGLU 118 and 119).
+double packed_tile_us(int M, int K, int N, int num_cus, bool swiglu) {
+    const int cus = num_cus > 0 ? num_cus : 256;
+    return with_tile<true>(M, K, N, cus, 1, [&](auto tile) {
+        using C = decltype(tile);
+        return tile_us<C>(M, K, N, cus, C::BM == 128 ? (swiglu ? 5.0 : 2.0) : swiglu ? 1.5 : 1.0);
+    });
+}
+
+TileShape tile_shape(int M, int K, int N, int num_cus, int kranges, bool packed_out) {
+    auto shape = [](auto tile) {
+        using C = decltype(tile);
+        return TileShape{C::KG, C::BM, C::BN};
+    };
+    return packed_out ? with_tile<true>(M, K, N, num_cus, kranges, shape)
+                      : with_tile<false>(M, K, N, num_cus, kranges, shape);
+}
+
+template <int EPI>
+static hipError_t tile_gemm_t(const void *packed, const uint8_t *w, int K, int N, int M, float *out, int64_t ldo,
+                              int32_t *nonfinite, int num_cus, int kranges, const GemmEpi &epi, hipStream_t s) {
+    return with_tile<EPI == 3>(M, K, N, num_cus, kranges, [&](auto tile) {
+        return launch_tile<decltype(tile), EPI>(packed, w, K, N, M, out, ldo, nonfinite, epi, s);
+    });
 }
 
 hipError_t launch_tile_gemm(const void *packed, const uint8_t *w, int K, int N, int M, float *out, int64_t ldo,

@@ -18,3 +18,25 @@ def oracle():
     from oracle import b1_oracle
     b1_oracle.lib()  # builds oracle/_build/libb1oracle.so if it is missing
     return b1_oracle
+
+
+KINDS = {"plain": (0, 0), "gate_residual": (1, 0), "swiglu": (2, 0), "packed": (3, 0), "packed_gelu": (3, 1),
+         "packed_swiglu": (3, 2)}
+
+
+@pytest.fixture(scope="session")
+def gemm_plan():
+    """gemm_plan(m, k, n, epilogue="plain", split=0): the name of the kernel a
+    packed GEMM of that shape runs on 256 CUs (no device needed)."""
+    import ctypes
+
+    import bonsai_b1
+    lib = bonsai_b1.load()
+
+    def plan(m, k, n, epilogue="plain", split=0):
+        kind, act = KINDS[epilogue]
+        name = ctypes.create_string_buffer(32)
+        lib.b1_gemm_plan(m, k, n, 256, kind, act, split, name, ctypes.c_size_t(len(name)))
+        return name.value.decode()
+
+    return plan

@@ -1,0 +1,27 @@
+"""Which kernel a packed GEMM runs (on the CPU: the rules take a shape and a CU
+count)."""
+import pytest
+
+# (m, k, n, epilogue, split): us on an MI355X with the persistent kernel and
+# with the faster of the one-range tiles of 64 x 192 and 128 x 192
+MEASURED = [
+    (4592, 3072, 12288, "plain", 0, 319.8, 303.5), (4000, 3072, 9216, "plain", 0, 219.6, 203.6),
+    (2200, 3072, 3072, "plain", 0, 60.2, 51.5), (1024, 3072, 18432, "plain", 0, 123.7, 110.7),
+    (4096, 3072, 12288, "plain", 0, 260.9, 269.9), (4240, 3072, 9216, "plain", 0, 221.8, 225.0),
+    (4608, 15360, 3072, "plain", 0, 326.2, 421.0), (3840, 3072, 3072, "plain", 0, 63.0, 68.4),
+    (2200, 3072, 3072, "gate_residual", 0, 65.6, 55.0), (1500, 9216, 3072, "gate_residual", 0, 201.5, 107.9),
+    (2836, 1152, 24640, "gate_residual", 0, 233.9, 242.8), (3968, 1536, 26304, "gate_residual", 0, 391.4, 408.1),
+    (3000, 3072, 18432, "swiglu", 0, 309.3, 300.9), (2200, 3072, 18432, "swiglu", 0, 227.0, 233.0),
+    (4592, 3072, 12288, "packed_swiglu", 0, 310.2, 318.5), (3744, 768, 19456, "packed_swiglu", 6464, 126.3, 146.6),
+    (4498, 768, 8896, "packed_swiglu", 0, 77.9, 87.4), (3808, 2688, 22528, "packed_swiglu", 7488, 411.4, 447.0),
+    (1600, 768, 7104, "packed_swiglu", 0, 25.1, 31.5), (594, 1152, 15488, "packed_swiglu", 5120, 30.5, 36.4),
+    (3300, 3072, 21504, "packed_gelu", 9216, 385.7, 394.8), (3773, 768, 15040, "packed_gelu", 0, 107.1, 108.8),
+    (1024, 3072, 18432, "packed_swiglu", 0, 125.7, 118.2),
+]
+
+
+@pytest.mark.parametrize("m,k,n,epilogue,split,persistent,tiles", MEASURED)
+def test_picks_the_faster_kernel(gemm_plan, m, k, n, epilogue, split, persistent, tiles):
+    name = gemm_plan(m, k, n, epilogue, split)
+    us = tiles if name.startswith("k1 ") else persistent
+    assert us <= 1.03 * min(persistent, tiles), name
