@@ -123,6 +123,8 @@ hipError_t launch_gemm_packed_epi(const void *packed, const uint8_t *w, int K, i
 // the kernel that they are about; no part of the C ABI.
 extern "C" void b1_gemm_plan(int M, int K, int N, int num_cus, int kind, int act, int split, char *name,
                              size_t size);
+// The same for the fused-conversion GEMM: its tile, "<rows>x<columns>".
+extern "C" void b1_fused_plan(int M, int K, int N, int num_cus, char *name, size_t size);
 
 // The epilogue (kind 1 or 2) as a separate pass over y [M][ldy] (N columns
 // of y; kind 2 writes glu_h of them).

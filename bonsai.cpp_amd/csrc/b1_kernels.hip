@@ -32,6 +32,7 @@
 // unchanged.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 #include <mutex>
 
@@ -3829,29 +3830,50 @@ extern "C" void b1_gemm_plan(int M, int K, int N, int num_cus, int kind, int act
 // The fused-conversion GEMM's tile by a time model: a launch of q tiles a CU
 // (rounded up) takes q times what one adds to a busy CU per 64 of K, or what
 // one takes alone if that is longer.  us per 64 of K, measured over 17 to
-// 4096 tokens: 128 x 512 2.65 and 1.9, 64 x 256 0.80 and 0.95, 64 x 128 0.47
-// and 0.75, 32 x 64 0.19 and 0.58 (M=4096 K=2048 N=8192: 172 us with 128 x
+// 4096 tokens: 64 x 256 0.80 and 0.95, 64 x 128 0.47 and 0.75, 32 x 64 0.19
+// and 0.58; 128 x 512, one work-group a CU, 2.2 and 12 us a tile for its
+// epilogue, a single tile 1.8 and 8 (M=4096 K=2048 N=8192: 172 us with 128 x
 // 512, 208 with 64 x 256, 243 with 64 x 128; M=1000 N=5504: 61, 41 and 40;
-// M=300 K=4096 N=1027: 100, 53, 44, and 34 with 32 x 64).
-static hipError_t launch_fused(const LinearArgs &a, int num_cus, hipStream_t s) {
+// M=300 K=4096 N=1027: 100, 53, 44, and 34 with 32 x 64; M=599 K=3968 N=14704,
+// one 128 x 512 tile a CU, 115, 118 and 135; M=2269 K=7488 N=9472, two, 421,
+// 439 and 506).  run(tile) with it.
+template <int BM_, int BN_, int WM_, int WN_>
+struct FusedTile {
+    static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_;
+};
+template <class Run>
+static auto with_fused_tile(int M, int K, int N, int num_cus, Run run) {
     const int64_t cus = num_cus > 0 ? num_cus : 256;
-    auto tiles = [&](int bm, int bn) {
-        return ((a.M + (int64_t)bm - 1) / bm) * ((a.N + (int64_t)bn - 1) / bn);
+    auto per_cu = [&](int bm, int bn) {
+        const int64_t tiles = ((M + (int64_t)bm - 1) / bm) * ((N + (int64_t)bn - 1) / bn);
+        return (double)((tiles + cus - 1) / cus);
     };
-    auto us = [&](int bm, int bn, double add, double alone) {
-        const double busy = (double)((tiles(bm, bn) + cus - 1) / cus) * add;
-        return busy > alone ? busy : alone;
-    };
-    const double t512 = us(128, 512, 2.65, 1.9), t256 = us(64, 256, 0.80, 0.95), t128 = us(64, 128, 0.47, 0.75),
-                 t64 = us(32, 64, 0.19, 0.58);
-    auto go = [&](auto kernel, int bm, int bn, int threads) {
-        hipLaunchKernelGGL(kernel, dim3((unsigned)tiles(bm, bn)), dim3(threads), 0, s, a, (a.N + bn - 1) / bn);
+    const double q512 = per_cu(128, 512), k64 = K / 64.0;
+    const double t512 = q512 > 1 ? q512 * (2.2 + 12.0 / k64) : 1.8 + 8.0 / k64,
+                 t256 = std::max(per_cu(64, 256) * 0.80, 0.95), t128 = std::max(per_cu(64, 128) * 0.47, 0.75),
+                 t64 = std::max(per_cu(32, 64) * 0.19, 0.58);
+    if (t512 <= t256 && t512 <= t128 && t512 <= t64) return run(FusedTile<128, 512, 128, 64>{});
+    if (t256 <= t128 && t256 <= t64) return run(FusedTile<64, 256, 64, 64>{});
+    if (t128 <= t64) return run(FusedTile<64, 128, 64, 32>{});
+    return run(FusedTile<32, 64, 32, 32>{});
+}
+
+static hipError_t launch_fused(const LinearArgs &a, int num_cus, hipStream_t s) {
+    return with_fused_tile(a.M, a.K, a.N, num_cus, [&](auto tile) {
+        using T = decltype(tile);
+        const int tiles_m = (int)((a.M + (int64_t)T::BM - 1) / T::BM),
+                  tiles_n = (int)((a.N + (int64_t)T::BN - 1) / T::BN);
+        hipLaunchKernelGGL((b1_gemm_fused_kernel<T::BM, T::BN, T::WM, T::WN>),
+                           dim3((unsigned)((int64_t)tiles_m * tiles_n)),
+                           dim3((T::BM / T::WM) * (T::BN / T::WN) * 64), 0, s, a, tiles_n);
         return hipGetLastError();
-    };
-    if (t512 <= t256 && t512 <= t128 && t512 <= t64) return go(b1_gemm_fused_kernel<128, 512, 128, 64>, 128, 512, 512);
-    if (t256 <= t128 && t256 <= t64) return go(b1_gemm_fused_kernel<64, 256, 64, 64>, 64, 256, 256);
-    if (t128 <= t64) return go(b1_gemm_fused_kernel<64, 128, 64, 32>, 64, 128, 256);
-    return go(b1_gemm_fused_kernel<32, 64, 32, 32>, 32, 64, 128);
+    });
+}
+
+extern "C" void b1_fused_plan(int M, int K, int N, int num_cus, char *name, size_t size) {
+    with_fused_tile(M, K, N, num_cus, [&](auto tile) {
+        snprintf(name, size, "%dx%d", decltype(tile)::BM, decltype(tile)::BN);
+    });
 }
 
 hipError_t launch_gemm(const LinearArgs &a, int num_cus, void *workspace, size_t ws_bytes, hipStream_t s) {

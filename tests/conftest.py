@@ -40,3 +40,20 @@ def gemm_plan():
         return name.value.decode()
 
     return plan
+
+
+@pytest.fixture(scope="session")
+def fused_plan():
+    """fused_plan(m, k, n): the tile of the GEMM that converts fp32 activations
+    itself, on 256 CUs."""
+    import ctypes
+
+    import bonsai_b1
+    lib = bonsai_b1.load()
+
+    def plan(m, k, n):
+        name = ctypes.create_string_buffer(32)
+        lib.b1_fused_plan(m, k, n, 256, name, ctypes.c_size_t(len(name)))
+        return name.value.decode()
+
+    return plan

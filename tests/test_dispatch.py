@@ -1,5 +1,4 @@
-"""Which kernel a packed GEMM runs (on the CPU: the rules take a shape and a CU
-count)."""
+"""Which kernel a GEMM runs (on the CPU: the rules take a shape and a CU count)."""
 import pytest
 
 # (m, k, n, epilogue, split): us on an MI355X with the persistent kernel and
@@ -25,3 +24,29 @@ def test_picks_the_faster_kernel(gemm_plan, m, k, n, epilogue, split, persistent
     name = gemm_plan(m, k, n, epilogue, split)
     us = tiles if name.startswith("k1 ") else persistent
     assert us <= 1.03 * min(persistent, tiles), name
+
+
+# (m, k, n): us with the fused-conversion GEMM's tiles of 128 x 512, 64 x 256,
+# 64 x 128 and 32 x 64
+FUSED = [
+    (599, 3968, 14704, 114.9, 117.7, 135.3, 190.2),
+    (4484, 3648, 2176, 107.8, 103.2, 123.2, 181.6),
+    (2884, 4544, 4096, 130.8, 142.1, 167.9, 269.3),
+    (3531, 4160, 2816, 120.4, 117.6, 140.5, 207.6),
+    (2269, 7488, 9472, 420.9, 438.9, 505.7, 838.4),
+    (2752, 256, 3968, 21.7, 17.8, 19.6, 20.6),
+    (738, 576, 15488, 31.3, 27.7, 31.1, 38.5),
+    (3753, 3968, 1792, 109.6, 74.2, 99.4, 135.6),
+    (572, 1856, 10240, 58.8, 38.5, 39.4, 64.1),
+    (1582, 1344, 1928, 42.4, 22.7, 20.3, 27.7),
+    (1756, 192, 3840, 18.6, 12.9, 12.4, 12.9),
+    (273, 1024, 3336, 34.1, 16.9, 13.0, 11.5),
+    (29, 192, 10208, 10.8, 7.5, 6.3, 6.2),
+]
+
+
+@pytest.mark.parametrize("m,k,n,t512,t256,t128,t64", FUSED)
+def test_picks_the_faster_tile(fused_plan, m, k, n, t512, t256, t128, t64):
+    us = dict(zip(("128x512", "64x256", "64x128", "32x64"), (t512, t256, t128, t64)))
+    name = fused_plan(m, k, n)
+    assert us[name] <= 1.05 * min(us.values()), name
