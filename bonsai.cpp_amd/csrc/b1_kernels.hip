@@ -263,6 +263,70 @@ struct GemmCfg {
     static_assert(WM % 32 == 0 && WN % 32 == 0, "32x32 sub-tiles");
 };
 
+// The sums of R rows (row: their addresses, in scalar registers) over one
+// column's packed weights wr, with b1_exact_kernel's steps: activations by
+// scalar loads, KS elements a row one step ahead, fp16 sign pairs, a block's
+// weights read a block ahead, or 4 for one row, whose block takes less than a
+// load.
+template <int R, int KS>
+__device__ __forceinline__ void exact_rows(uint64_t (&row)[R], const uint16_t *wr, int K, float (&sum)[R]) {
+#pragma clang fp contract(off)
+    typedef float row_v __attribute__((ext_vector_type(KS), aligned(4)));
+    typedef const __attribute__((address_space(4))) row_v const_row;
+    row_v next[R];
+    auto load = [&](uint32_t off) {
+        asm volatile("" : "+s"(off)); // (keeps the loads of several steps apart)
+#pragma unroll
+        for (int r = 0; r < R; ++r) next[r] = *(const_row *)(row[r] + off);
+    };
+#pragma unroll
+    for (int r = 0; r < R; ++r) sum[r] = 0.0f;
+    load(0);
+    const int last = K / 32 - 1;
+    constexpr int D = R == 1 ? 4 : 1;
+    uint32_t q[D][3]; // the weights of blocks b .. b + D - 1
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+#pragma unroll
+        for (int i = 0; i < 3; ++i) q[d][i] = wr[3 * min(d, last) + i];
+    for (int b = 0; b <= last; ++b) {
+        const float scale = (float)__builtin_bit_cast(_Float16, (uint16_t)q[0][0]);
+        const uint32_t bits = q[0][1] | q[0][2] << 16;
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+#pragma unroll
+            for (int d = 0; d + 1 < D; ++d) q[d][i] = q[d + 1][i];
+            q[D - 1][i] = wr[3 * min(b + D, last) + i];
+        }
+        float bs[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) bs[r] = 0.0f;
+#pragma unroll
+        for (int i0 = 0; i0 < 32; i0 += KS) {
+            // scalar loads return out of order: wait for this step's before
+            // the next step's are issued
+            wait_lgkmcnt0();
+            __builtin_amdgcn_sched_barrier(0);
+            row_v a[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) a[r] = next[r];
+            load(i0 + KS < 32 ? 128u * b + 4 * (i0 + KS) : 128u * min(b + 1, last));
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < KS; ++j) {
+                const int i = i0 + j;
+                // +1.0 for a set bit, -1.0 for a clear one
+                const half2v sg = __builtin_bit_cast(half2v, ((bits << (15 - (i & 15))) & kSignPair) ^ 0xBC00BC00u);
+#pragma unroll
+                for (int r = 0; r < R; ++r) bs[r] = __builtin_fmaf(a[r][j], (float)sg[i >> 4], bs[r]);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int r = 0; r < R; ++r) sum[r] = sum[r] + scale * bs[r];
+    }
+}
+
 // The GEMM that converts fp32 activations while it stages each tile, for
 // calls without a packing (no workspace, or K no multiple of 384).  A tile
 // reads its rows once per column tile and its weights once per row tile, 4
@@ -274,15 +338,23 @@ struct GemmCfg {
 //
 // A row holding an |a| >= 65520 (or an inf), which fp16 cannot take, is not
 // stored from the tile: the work-group, which has seen all of the row,
-// computes its columns in the reference's scalar order, the arithmetic of
-// b1_exact_kernel, so its outputs are EXACT mode's bit for bit.  (A second
-// launch that read every row again to find them took 5 us at M=1000.)
+// computes its columns in the reference's scalar order (exact_rows, 4 such
+// rows and 64 columns a wave at a time), so its outputs are EXACT mode's bit
+// for bit.  (A second launch that read every row again to find them took 5 us
+// at M=1000.)  us with every row beyond fp16, one output a thread at a time ->
+// now (a second launch, a work-group a row): M=92 K=1472 N=1552 270 -> 92
+// (216), M=308 K=2496 N=272 670 -> 151 (145), M=518 K=2112 N=160, few tiles,
+// 416 -> 129 (92); one row of M=965 K=2048 N=3032 52 -> 45 (497).  The branch
+// is marked unlikely, and tiles of one or two rows of sub-tiles read both
+// halves of a block's fragments ahead by themselves: otherwise its scalar
+// registers and the compiler's schedule for them come out of the stage loop
+// (31.0 us -> 32.3 at M=582 K=5312 N=128).
 template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kernel(LinearArgs p, int tiles_n) {
     using C = GemmCfg<BM, BN, WM, WN>;
     __shared__ __attribute__((aligned(16))) uint8_t lds[2 * C::STAGE];
     __shared__ uint32_t over[BM]; // rows beyond the fp16 range
-    static_assert(BM <= C::NT, "one thread a row clears the flags");
+    static_assert(BM <= C::NT && BM <= 128, "one thread a row clears the flags, two masks hold them");
 
     const int t = xcd_tile(blockIdx.x, gridDim.x);
     const int tm = t / tiles_n, tn = t - tm * tiles_n;
@@ -378,18 +450,26 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kern
             u32x4 wb[C::NTL][2];
 #pragma unroll
             for (int nt = 0; nt < C::NTL; ++nt) wpair_quads<0>(wg[nt], wg[nt] >> 8, s2[nt], wb[nt][0], wb[nt][1]);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                half8 af[C::MT];
+            half8 af[2][C::MT];
+            auto read = [&](int h) {
 #pragma unroll
                 for (int mt = 0; mt < C::MT; ++mt)
-                    af[mt] = *reinterpret_cast<const half8 *>(base + mt * 32 * C::ROW + b * 64 + h * 32);
+                    af[h][mt] = *reinterpret_cast<const half8 *>(base + mt * 32 * C::ROW + b * 64 + h * 32);
+            };
+            if constexpr (C::MT <= 2) {
+                read(0);
+                read(1);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                if constexpr (C::MT > 2) read(h);
 #pragma unroll
                 for (int nt = 0; nt < C::NTL; ++nt) {
                     const half8 bf = __builtin_bit_cast(half8, wb[nt][h]);
 #pragma unroll
                     for (int mt = 0; mt < C::MT; ++mt)
-                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[mt], bf, acc[mt][nt], 0, 0, 0);
+                        acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(af[h][mt], bf, acc[mt][nt], 0, 0, 0);
                 }
             }
         }
@@ -443,27 +523,52 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void b1_gemm_fused_kern
             }
         }
     }
-    if (any) {
-#pragma clang fp contract(off)
-        for (int e = tid; e < BM * BN; e += C::NT) {
-            const int r = e / BN, m = m0 + r, n = n0 + e - r * BN;
-            if (!over[r] || m >= p.M || n >= p.N) continue;
-            const float *xr = p.act + (size_t)m * p.lda;
-            const uint16_t *wr = reinterpret_cast<const uint16_t *>(p.w + (size_t)n * rs);
-            float sum = 0.0f;
-            for (int b = 0; b < p.K / 32; ++b) {
-                const float scale = (float)__builtin_bit_cast(_Float16, wr[3 * b]);
-                const uint32_t bits = (uint32_t)wr[3 * b + 1] | ((uint32_t)wr[3 * b + 2] << 16);
-                float bs = 0.0f;
-                for (int i4 = 0; i4 < 32; i4 += 4) {
-                    const floatx4 a = *reinterpret_cast<const floatx4 *>(xr + 32 * b + i4);
+    if (__builtin_expect(any, 0)) {
+        uint64_t rows[2];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) bs = ((bits >> (i4 + j)) & 1u) ? bs + a[j] : bs - a[j];
+        for (int h = 0; h < 2; ++h)
+            rows[h] = __builtin_amdgcn_ballot_w64(64 * h + lane < BM && over[min(64 * h + lane, BM - 1)] != 0);
+        const int w = __builtin_amdgcn_readfirstlane(wave);
+        for (int task = 0; rows[0] | rows[1];) {
+            int m[4], count = 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int h = rows[0] ? 0 : 1;
+                m[r] = r ? m[0] : 0;
+                if (rows[h]) {
+                    m[r] = m0 + 64 * h + __builtin_ctzll(rows[h]);
+                    rows[h] &= rows[h] - 1;
+                    ++count;
                 }
-                sum = sum + scale * bs;
             }
-            bad += !__builtin_isfinite(sum);
-            p.out[(size_t)m * p.ldo + n] = sum;
+            for (int c = 0; c < BN / 64; ++c, ++task) {
+                if (task % C::NW != w) continue;
+                const int n = n0 + 64 * c + lane;
+                const uint16_t *wr = reinterpret_cast<const uint16_t *>(p.w + (size_t)min(n, p.N - 1) * rs);
+                uint64_t row[4];
+                float sum[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    row[r] = reinterpret_cast<uint64_t>(p.act + (size_t)m[r] * p.lda);
+                    asm volatile("" : "+s"(row[r]));
+                }
+                if (count > 1) {
+                    exact_rows<4, 8>(row, wr, p.K, sum);
+                } else {
+                    uint64_t row1[1] = {row[0]};
+                    float sum1[1];
+                    exact_rows<1, 32>(row1, wr, p.K, sum1);
+                    sum[0] = sum1[0];
+                }
+                if (n < p.N) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (r < count) {
+                            bad += !__builtin_isfinite(sum[r]);
+                            p.out[(size_t)m[r] * p.ldo + n] = sum[r];
+                        }
+                }
+            }
         }
     }
     count_nonfinite(p.nonfinite, bad);

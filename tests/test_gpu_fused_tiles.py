@@ -73,3 +73,30 @@ def test_tiles(torch, b1, m, k, n):
     assert torch.equal(z[big], e[big])
     assert bool(torch.isnan(z[m - 2]).all())
     assert int(nf.item()) == int((~torch.isfinite(z)).sum())
+
+
+@pytest.mark.parametrize("m,k,n", [(17, 64, 1), (77, 2048, 130), (33, 448, 65), (640, 128, 4097), (1000, 192, 8100),
+                                   (2000, 448, 8100)])
+@pytest.mark.parametrize("step", [1, 3])
+def test_many_rows_beyond_fp16(torch, b1, m, k, n, step):
+    """Every row, or every third one, beyond the fp16 range: whole groups of 4
+    flagged rows a wave, the remainders of a tile's flagged rows and of its
+    columns, at every tile; EXACT mode's bits in those rows, the others
+    unchanged."""
+    from bonsai_b1 import synth
+    print(f"fused gemm, rows beyond fp16 ({m},{k},{n}) step {step}", flush=True)
+    a = synth.device_activations(m, k, 53)
+    w = synth.device_packed_weights(n, k, 54)
+    y = b1.linear(a, w, n, mode="gemm")
+    big = torch.arange(0, m, step, device="cuda")
+    a[big] *= 1.0e6
+    nf = torch.zeros(1, dtype=torch.int32, device="cuda")
+    buf = torch.full((m, n + 3), 7.0, device="cuda")
+    b1.linear(a, w, n, out=buf[:, :n], mode="gemm", nonfinite=nf)
+    e = b1.linear(a, w, n, mode="exact")
+    torch.cuda.synchronize()
+    keep = torch.ones(m, dtype=torch.bool, device="cuda")
+    keep[big] = False
+    assert torch.equal(buf[big, :n], e[big])
+    assert torch.equal(buf[keep, :n], y[keep])
+    assert bool((buf[:, n:] == 7.0).all()) and int(nf.item()) == 0
