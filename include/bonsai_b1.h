@@ -219,7 +219,17 @@ int bonsai_b1_pack_act_f16_ld(const float *act, int64_t lda, int in_dim,
  * activations within the fp16 range).  Allocates nothing.  The _ws form
  * accepts a workspace of bonsai_b1_linear_packed_workspace_bytes bytes,
  * which earlier versions needed for K split over work-groups; it runs the
- * same kernels with the same results without one. */
+ * same kernels with the same results without one.
+ *
+ * The bits of a row: the packed GEMM (this entry, its epilogue, _to_packed and
+ * _scaled forms, the fp32 entries over a packing, and batches) sums K in one
+ * range, or where there are few output tiles in 2, 4 or 8 ranges added in
+ * order.  How many follows batch, in_dim and out_dim alone, so that all these
+ * entries give a linear the same y; a call over some of its rows may sum
+ * another number of ranges, the same values up to the order of fp32 sums.
+ * From ceil(batch / 64) * ceil(out_dim / 192) >= 1.25 times the device's CUs
+ * (320 on 256) it is one range, and a row's bits depend on neither the rows
+ * with it nor the kernel. */
 int bonsai_b1_linear_packed_f16(const void *packed_act, const void *w,
                                 int in_dim, int out_dim, int batch,
                                 float *out, int64_t ldo, int32_t *nonfinite,
@@ -464,7 +474,8 @@ int bonsai_b1_linear_packed_f16_epi(const void *packed_act, const void *w,
  * out_dim - split); in_dim % 384 == 0; split > 0: out 16-byte aligned,
  * ldo >= split, ldo % 4 == 0; packed columns: packed_out 16-byte aligned,
  * ldp >= their count, ldp % 8 == 0; the outputs apart from packed_act and
- * from each other.  Always the 128-row GEMM tile, also for a few rows.
+ * from each other.  Always the packed GEMM, also for a few rows (where
+ * bonsai_b1_linear_packed_f16 takes its small-M kernel).
  * No reference counterpart as one op (the reference runs separate ggml ops).
  */
 enum {

@@ -57,3 +57,18 @@ def fused_plan():
         return name.value.decode()
 
     return plan
+
+
+@pytest.fixture(scope="session")
+def unpack():
+    """unpack(raw, n, k): float64 [n, k] of packed B1_0 weights on the GPU."""
+    import torch
+
+    def weights(raw, n, k):
+        blocks = raw.reshape(n, k // 32, 6)
+        scale = blocks[:, :, :2].contiguous().view(torch.float16).double()
+        bits = torch.arange(8, device=raw.device, dtype=torch.uint8)
+        sign = 2.0 * ((blocks[:, :, 2:].unsqueeze(-1) >> bits) & 1).double() - 1.0
+        return (sign.reshape(n, k // 32, 32) * scale).reshape(n, k)
+
+    return weights

@@ -34,16 +34,8 @@ def b1(torch):
     return bonsai_b1
 
 
-def unpack(torch, raw, n, k):
-    blocks = raw.reshape(n, k // 32, 6)
-    scale = blocks[:, :, :2].contiguous().view(torch.float16).double()
-    bits = torch.arange(8, device=raw.device, dtype=torch.uint8)
-    sign = 2.0 * ((blocks[:, :, 2:].unsqueeze(-1) >> bits) & 1).double() - 1.0
-    return (sign.reshape(n, k // 32, 32) * scale).reshape(n, k)
-
-
 @pytest.mark.parametrize("m,k,n", SHAPES)
-def test_tiles(torch, b1, m, k, n):
+def test_tiles(torch, b1, unpack, m, k, n):
     from bonsai_b1 import synth
     print(f"fused gemm ({m},{k},{n})", flush=True)
     a = synth.device_activations(m, k, 51)
@@ -53,7 +45,7 @@ def test_tiles(torch, b1, m, k, n):
     torch.cuda.synchronize()
     y = buf[:, :n].clone()
     assert bool((buf[:, n:] == 7.0).all())
-    h, wd = a.half().double(), unpack(torch, w, n, k)
+    h, wd = a.half().double(), unpack(w, n, k)
     ref, mag = h @ wd.t(), h.abs() @ wd.abs().t()
     assert float(((y.double() - ref).abs() / (2.0 * k * 2.0 ** -24 * mag)).max()) <= 1.0
     # rows beyond the fp16 range, first, last and at a tile's edge

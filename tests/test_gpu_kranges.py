@@ -50,16 +50,8 @@ def b1(torch):
     return bonsai_b1
 
 
-def unpack(torch, raw, n, k):
-    blocks = raw.reshape(n, k // 32, 6)
-    scale = blocks[:, :, :2].contiguous().view(torch.float16).double()
-    bits = torch.arange(8, device=raw.device, dtype=torch.uint8)
-    sign = 2.0 * ((blocks[:, :, 2:].unsqueeze(-1) >> bits) & 1).double() - 1.0
-    return (sign.reshape(n, k // 32, 32) * scale).reshape(n, k)
-
-
 @pytest.mark.parametrize("m,k,n", SHAPES)
-def test_plain(torch, b1, m, k, n):
+def test_plain(torch, b1, unpack, m, k, n):
     from bonsai_b1 import synth
     say(f"k-range gemm ({m},{k},{n})")
     a = synth.device_activations(m, k, 401)
@@ -72,7 +64,7 @@ def test_plain(torch, b1, m, k, n):
     assert torch.equal(out[:, :n], y) and bool((out[:, n:] == 7.0).all())
     assert int(nf.item()) == 0
     h = a.half().double()
-    wd = unpack(torch, w, n, k)
+    wd = unpack(w, n, k)
     ref, mag = h @ wd.t(), h.abs() @ wd.abs().t()
     over = ((y.double() - ref).abs() / (2.0 * k * 2.0 ** -24 * mag)).max()
     say(f"  largest error / bound {float(over):.3e}")

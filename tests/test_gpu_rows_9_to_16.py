@@ -27,24 +27,16 @@ def b1(torch):
     return bonsai_b1
 
 
-def unpack(torch, raw, n, k):
-    blocks = raw.reshape(n, k // 32, 6)
-    scale = blocks[:, :, :2].contiguous().view(torch.float16).double()
-    bits = torch.arange(8, device=raw.device, dtype=torch.uint8)
-    sign = 2.0 * ((blocks[:, :, 2:].unsqueeze(-1) >> bits) & 1).double() - 1.0
-    return (sign.reshape(n, k // 32, 32) * scale).reshape(n, k)
-
-
 @pytest.mark.parametrize("m,k,n", [(9, 256, 1), (10, 1024, 300), (12, 3072, 9216), (13, 3328, 97), (15, 9216, 600),
                                    (16, 3072, 4100), (16, 512, 17)])
-def test_rows(torch, b1, m, k, n):
+def test_rows(torch, b1, unpack, m, k, n):
     from bonsai_b1 import synth
     print(f"small batch ({m},{k},{n})", flush=True)
     a = torch.zeros((m, k + 4), device="cuda")[:, :k]      # rows apart
     a.copy_(synth.device_activations(m, k, 71))
     w = synth.device_packed_weights(n, k, 72)
     y = b1.linear(a, w, n, mode="gemv")
-    h, wd = a.half().double(), unpack(torch, w, n, k)
+    h, wd = a.half().double(), unpack(w, n, k)
     ref, mag = h @ wd.t(), h.abs() @ wd.abs().t()
     torch.cuda.synchronize()
     assert float(((y.double() - ref).abs() / (2.0 * k * 2.0 ** -24 * mag)).max()) <= 1.0
