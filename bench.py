@@ -157,8 +157,8 @@ def bench_tiles16(torch, b1, synth, steps, warmup):
 def bench_step_kernels(torch, b1, a, w, n, steps, warmup):
     """The two kernels of the step, each timed alone with HIP events on its
     launch stream: the GEMM kernel over packed activations
-    (bonsai_b1_linear_packed_f16_scaled: b1_gemm_kernel alone at an unsplit
-    shape) and the range-safe pack pass (bonsai_b1_pack_act_f16_scaled:
+    (bonsai_b1_linear_packed_f16_scaled: b1_gemm_kernel alone at the
+    headline shape) and the range-safe pack pass (bonsai_b1_pack_act_f16_scaled:
     b1_pack_rows_kernel alone).  Returns (gemm ms, pack ms)."""
     m, k = a.shape
     packed, rs = b1.pack_act_f16_scaled(a)
@@ -470,8 +470,7 @@ def bench_c4_mlp(torch, b1, synth, reps=4):
 
 def bench_configs(torch, b1, synth, steps, warmup):
     """The other config shapes, each from fp32 activations through
-    bonsai_b1_linear_f32 (pack pass + GEMM; split along K where the shape
-    asks for it): C1 (256 x 3072 -> 3072), C3 q/k/v and out-projection,
+    bonsai_b1_linear_f32 (pack pass + GEMM): C1 (256 x 3072 -> 3072), C3 q/k/v and out-projection,
     C4 up- and down-projection, GELU-tanh between them, and the C4 chain in
     its fused form (GELU in the up-projection's epilogue, written as the
     down-projection's packed input); then the C5 38-block step."""

@@ -125,6 +125,8 @@ extern "C" void b1_gemm_plan(int M, int K, int N, int num_cus, int kind, int act
                              size_t size);
 // The same for the fused-conversion GEMM: its tile, "<rows>x<columns>".
 extern "C" void b1_fused_plan(int M, int K, int N, int num_cus, char *name, size_t size);
+// The rows an EXACT work-group takes.
+extern "C" int b1_exact_plan(int M, int N, int num_cus);
 
 // The epilogue (kind 1 or 2) as a separate pass over y [M][ldy] (N columns
 // of y; kind 2 writes glu_h of them).

@@ -3561,41 +3561,43 @@ __global__ __launch_bounds__(kGvWaves * 64, WL == kG4WL2 ? 4 : 2) void b1_gemv_g
 
 // ------------------------------------------------------------- launchers --
 
-hipError_t launch_exact(const LinearArgs &a, int num_cus, hipStream_t s) {
-    // Rows TM a work-group shares its signs over: 4, 2 or 1.  A launch takes
-    // about q work-groups a CU (rounded up) times what one adds to a busy CU,
-    // or what one takes alone if that is longer; us at K = 3072: TM = 4 31.5
-    // and 38 (q = 3, M=256 N=3072: 94), TM = 2 17.4 and 22, TM = 1 11.8 and
-    // 15 (q = 1, M=7 N=3072: 15.1, against 22 with TM = 2 and 38 with 4).
-    const int64_t cus = num_cus > 0 ? num_cus : 256, cols = (a.N + kExTN - 1) / kExTN;
-    auto us = [&](int tm, double add, double alone) {
-        const int64_t wgs = cols * ((a.M + (int64_t)tm - 1) / tm);
-        const double busy = (double)((wgs + cus - 1) / cus) * add;
-        return busy > alone ? busy : alone;
+// Rows a work-group of the EXACT kernels shares its signs over: 4, 2 or 1
+// (b1_exact_kernel), or 16 or 8 through LDS (b1_exact_lds_kernel).  A launch
+// takes about q work-groups a CU (rounded up) times what one adds to a busy
+// CU, or what one takes alone if that is longer; us at K = 3072: 4 rows 31.5
+// and 38 (q = 3, M=256 N=3072: 94), 2 rows 17.4 and 22, 1 row 11.8 and 15 (q =
+// 1, M=7 N=3072: 15.1, against 22 with 2 rows and 38 with 4).  Through LDS
+// while that leaves at least 4 work-groups (16 waves) a CU (M=1024 K=3072
+// N=4768: 565 us, with 4 rows 611; M=4096 N=12288 4.96 ms, 5.99; M=256 N=3072,
+// below, 151 with 4 rows, 107).
+static int exact_rows_of(int M, int N, int num_cus) {
+    const int64_t cus = num_cus > 0 ? num_cus : 256, cols = (N + kExTN - 1) / kExTN;
+    auto wgs = [&](int64_t rows) { return cols * ((M + rows - 1) / rows); };
+    if (M > 8 && wgs(16) >= 4 * cus) return 16;
+    if (M > 4 && wgs(8) >= 4 * cus) return 8;
+    auto us = [&](int rows, double add, double alone) {
+        return std::max((double)((wgs(rows) + cus - 1) / cus) * add, alone);
     };
-    // 16 or 8 rows through LDS while that leaves at least 4 work-groups (16
-    // waves) a CU (M=1024 K=3072 N=4768: 565 us, with 4 rows 611; M=4096
-    // N=12288 4.96 ms, 5.99; M=256 N=3072, below, 151 with 4 rows, 107)
-    if (a.M > 8 && cols * ((a.M + 15) / 16) >= 4 * cus) {
-        hipLaunchKernelGGL((b1_exact_lds_kernel<16>), dim3((unsigned)cols, (unsigned)((a.M + 15) / 16)), dim3(kExTN), 0, s, a);
-        return hipGetLastError();
-    }
-    if (a.M > 4 && cols * ((a.M + 7) / 8) >= 4 * cus) {
-        hipLaunchKernelGGL((b1_exact_lds_kernel<8>), dim3((unsigned)cols, (unsigned)((a.M + 7) / 8)), dim3(kExTN), 0, s, a);
-        return hipGetLastError();
-    }
     const double us1 = us(1, 11.8, 15.0), us2 = us(2, 17.4, 22.0), us4 = us(4, 31.5, 38.0);
-    auto go = [&](auto kernel, int tm) {
-        const dim3 grid((unsigned)cols, (unsigned)((a.M + (int64_t)tm - 1) / tm));
+    return us1 <= us2 && us1 <= us4 ? 1 : us2 <= us4 ? 2 : 4;
+}
+
+extern "C" int b1_exact_plan(int M, int N, int num_cus) { return exact_rows_of(M, N, num_cus); }
+
+hipError_t launch_exact(const LinearArgs &a, int num_cus, hipStream_t s) {
+    const int rows = exact_rows_of(a.M, a.N, num_cus);
+    auto go = [&](auto kernel) {
+        const dim3 grid((unsigned)((a.N + kExTN - 1) / kExTN), (unsigned)((a.M + (int64_t)rows - 1) / rows));
         hipLaunchKernelGGL(kernel, grid, dim3(kExTN), 0, s, a);
+        return hipGetLastError();
     };
-    if (us1 <= us2 && us1 <= us4)
-        go(b1_exact_kernel<1, 32>, 1);
-    else if (us2 <= us4)
-        go(b1_exact_kernel<2, 16>, 2);
-    else
-        go(b1_exact_kernel<4, 8>, 4);
-    return hipGetLastError();
+    switch (rows) {
+    case 16: return go(b1_exact_lds_kernel<16>);
+    case 8: return go(b1_exact_lds_kernel<8>);
+    case 4: return go(b1_exact_kernel<4, 8>);
+    case 2: return go(b1_exact_kernel<2, 16>);
+    default: return go(b1_exact_kernel<1, 32>);
+    }
 }
 
 static bool fast_layout_ok(const LinearArgs &a) {

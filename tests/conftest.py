@@ -60,6 +60,14 @@ def fused_plan():
 
 
 @pytest.fixture(scope="session")
+def exact_plan():
+    """exact_plan(m, n): the rows an EXACT work-group takes on 256 CUs."""
+    import bonsai_b1
+    lib = bonsai_b1.load()
+    return lambda m, n: lib.b1_exact_plan(m, n, 256)
+
+
+@pytest.fixture(scope="session")
 def unpack():
     """unpack(raw, n, k): float64 [n, k] of packed B1_0 weights on the GPU."""
     import torch

@@ -204,7 +204,7 @@ def test_epilogue_workspace_bytes():
 
 
 def test_workspace_bytes_by_kernel():
-    """What each kernel choice needs (no device here, so no split-K): the
+    """What each kernel choice needs: the
     packed GEMM the range-safe packing; EXACT, the fused-conversion GEMM
     (K % 384 != 0) and the small-M kernel (which converts the activations
     itself) nothing."""
@@ -218,7 +218,7 @@ def test_workspace_bytes_by_kernel():
     assert lib.bonsai_b1_workspace_bytes(8, 3072, 18432, gemm) == pack_area(8, 3072)
     assert lib.bonsai_b1_workspace_bytes(8, 448, 64, auto) == 0
     assert lib.bonsai_b1_workspace_bytes(17, 3072, 64, gemv) == 0   # not a small-M batch
-    assert lib.bonsai_b1_linear_packed_workspace_bytes(256, 3072, 3072) == 0   # no device: unsplit
+    assert lib.bonsai_b1_linear_packed_workspace_bytes(256, 3072, 3072) == 0   # no device
 
 
 def test_norm_mod_rejects_before_device():

@@ -1,5 +1,34 @@
 """Which kernel a GEMM runs (on the CPU: the rules take a shape and a CU count)."""
+import importlib
+
 import pytest
+
+# Test modules whose shapes are there for one kernel each.
+PLANNED = ["test_gpu_kranges", "test_gpu_packed_out", "test_gpu_parity", "test_gpu_producers", "test_gpu_tiles16"]
+
+
+@pytest.mark.parametrize("module", PLANNED)
+def test_shapes_reach_their_kernels(gemm_plan, module):
+    for m, k, n, epilogue, split, name in importlib.import_module(f"tests.{module}").PLANS:
+        assert gemm_plan(m, k, n, epilogue, split) == name, (m, k, n, epilogue, split)
+
+
+def test_k_ranges(gemm_plan):
+    from tests import test_gpu_kranges as kranges
+    for ranges, shapes in kranges.RANGES.items():
+        for shape in shapes:
+            assert gemm_plan(*shape).startswith(f"k{ranges} "), shape
+
+
+def test_row_counts_and_fused_tiles_reach_their_kernels(exact_plan, fused_plan):
+    from tests import test_gpu_exact_rows as exact
+    from tests import test_gpu_fused_tiles as fused
+    for m, _, n, rows in exact.SHAPES + exact.NONFINITE:
+        assert exact_plan(m, n) == rows, (m, n)
+    assert {rows for *_, rows in exact.NONFINITE} == {1, 2, 4, 8, 16}
+    for m, k, n, tile in fused.SHAPES:
+        assert fused_plan(m, k, n) == tile, (m, k, n)
+
 
 # (m, k, n, epilogue, split): us on an MI355X with the persistent kernel and
 # with the faster of the one-range tiles of 64 x 192 and 128 x 192

@@ -8,7 +8,7 @@ the float64 SwiGLU, GELU-tanh and gate-residual of the reference graph,
 src/diffuser_graph.cpp:277-281,441-460,477-540), so a defect shared by the
 fused and the unfused path cannot pass:
 
-  * every op of a mixed batch (split-K fused q/k/v, SwiGLU, gate-residual in
+  * every op of a mixed batch (fused q/k/v, SwiGLU, gate-residual in
     place, packed GELU output, small-M, fused-conversion GEMM), each against
     the oracle on the inputs the GPU actually read;
   * the C3 out-projection, C4 down-projection and C5 linear2 shapes with the
@@ -94,7 +94,7 @@ def test_batch_ops_against_oracle(torch, b1, oracle):
     lib = b1.load()
     m, d = 512, 3072
     x = synth.device_activations(m, d, 301)
-    # q/k/v: three weights as adjacent row ranges (one split-K GEMM)
+    # q/k/v: three weights as adjacent row ranges (one GEMM)
     parts = [synth.device_packed_weights(1024, d, 302 + i) for i in range(3)]
     cs = (capi.B1WeightsC * 3)(*[b1.device_weights(p, d, 1024) for p in parts])
     cat = capi.B1WeightsC()

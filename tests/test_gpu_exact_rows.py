@@ -1,8 +1,8 @@
 """EXACT mode's kernel (b1_exact_kernel: 1, 2 or 4 rows a work-group, scalar
-activation loads, weights 4 blocks at a time; b1_exact_lds_kernel: 8 or 16) against the oracle's scalar
-order, bit for bit.
+activation loads, weights 4 blocks at a time; b1_exact_lds_kernel: 8 or 16)
+against the oracle's scalar order, bit for bit.
 
-Shapes: the three row counts on 256 CUs, row remainders, widths around the
+Shapes: the five row counts on 256 CUs, row remainders, widths around the
 256-column work-group, block counts around the groups of 4 (odd ones put the
 packed rows on 2-byte boundaries), and rows at strides and offsets that leave
 4-byte alignment only.  Values: N(0, 1), subnormals, signed zeros, and rows
@@ -15,12 +15,17 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [  # (m, k, n)
-    (1, 32, 1), (1, 3072, 257), (3, 96, 255), (5, 128, 513), (7, 160, 300),      # 1 row
-    (65, 224, 1000), (301, 64, 600), (130, 256, 769), (103, 416, 1024),          # 2 rows
-    (201, 288, 3000), (258, 1056, 1003), (1023, 192, 1500), (130, 128, 5000),    # 4 rows
-    (601, 96, 3600), (1030, 288, 4090),                                          # 8 and 16 (through LDS)
+SHAPES = [  # (m, k, n, rows a work-group on 256 CUs)
+    (1, 32, 1, 1), (1, 3072, 257, 1), (3, 96, 255, 1), (5, 128, 513, 1), (7, 160, 300, 1),
+    (65, 224, 1000, 2), (301, 64, 600, 2), (130, 256, 769, 2), (103, 416, 1024, 2), (201, 288, 3000, 2),
+    (258, 1056, 1003, 2),
+    # 4 rows: one quad of blocks and less, and K past 512, where lines are
+    # touched ahead inside the loop, with 1 and 3 blocks after the last quad
+    (1023, 192, 1500, 4), (130, 128, 5000, 4), (509, 672, 1500, 4), (1021, 608, 770, 4),
+    (601, 96, 3600, 8), (1030, 288, 4090, 16),          # through LDS
 ]
+NONFINITE = [(2, 96, 300, 1), (65, 224, 1000, 2), (258, 160, 3001, 2), (1021, 160, 770, 4), (601, 96, 3600, 8),
+             (1030, 96, 4090, 16)]
 
 
 @pytest.fixture(scope="module")
@@ -37,9 +42,10 @@ def b1(torch):
     return bonsai_b1
 
 
-@pytest.mark.parametrize("m,k,n", SHAPES)
-def test_bits(torch, b1, oracle, m, k, n):
+@pytest.mark.parametrize("m,k,n,rows", SHAPES)
+def test_bits(torch, b1, oracle, exact_plan, m, k, n, rows):
     from bonsai_b1 import synth
+    assert exact_plan(m, n) == rows
     print(f"exact ({m},{k},{n})", flush=True)
     sys.stdout.flush()
     act = synth.activations(m, k, 31 * m + k)
@@ -66,9 +72,10 @@ def test_bits(torch, b1, oracle, m, k, n):
     assert bool((out[:, n:] == 7.0).all()) and int(nf.item()) == 0
 
 
-@pytest.mark.parametrize("m,k,n", [(2, 96, 300), (65, 224, 1000), (258, 160, 3001)])
-def test_nonfinite(torch, b1, oracle, m, k, n):
+@pytest.mark.parametrize("m,k,n,rows", NONFINITE)
+def test_nonfinite(torch, b1, oracle, exact_plan, m, k, n, rows):
     from bonsai_b1 import synth
+    assert exact_plan(m, n) == rows
     print(f"exact non-finite ({m},{k},{n})", flush=True)
     act = synth.activations(m, k, 5)
     act[0, 9] = np.inf

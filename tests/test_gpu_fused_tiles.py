@@ -12,11 +12,11 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [  # (m, k, n), tile on 256 CUs
-    (17, 64, 1), (33, 448, 65), (77, 2048, 5504), (300, 320, 1027),   # 32 x 64
-    (1000, 256, 5500), (640, 128, 4097),                              # 64 x 128
-    (1000, 192, 8100), (1024, 64, 8193),                              # 64 x 256
-    (2000, 448, 8100), (2049, 64, 8192),                              # 128 x 512
+SHAPES = [  # (m, k, n, tile on 256 CUs)
+    (17, 64, 1, "32x64"), (33, 448, 65, "32x64"), (77, 2048, 5504, "32x64"), (300, 320, 1027, "32x64"),
+    (1000, 256, 5500, "64x128"), (640, 128, 4097, "64x128"), (1024, 64, 8193, "64x128"),
+    (1000, 192, 8100, "64x256"), (2049, 64, 8192, "64x256"),
+    (2000, 448, 8100, "128x512"), (2305, 896, 12300, "128x512"),
 ]
 
 
@@ -34,9 +34,10 @@ def b1(torch):
     return bonsai_b1
 
 
-@pytest.mark.parametrize("m,k,n", SHAPES)
-def test_tiles(torch, b1, unpack, m, k, n):
+@pytest.mark.parametrize("m,k,n,tile", SHAPES)
+def test_tiles(torch, b1, unpack, fused_plan, m, k, n, tile):
     from bonsai_b1 import synth
+    assert fused_plan(m, k, n) == tile
     print(f"fused gemm ({m},{k},{n})", flush=True)
     a = synth.device_activations(m, k, 51)
     w = synth.device_packed_weights(n, k, 52)

@@ -4,7 +4,8 @@ ranges and add the partial tiles in LDS.
 
 Shapes: every number of ranges and tile height on 256 CUs, row counts at and
 around the 32- and 64-row tile edges, widths one column past or short of a
-tile, K whose ranges are of unequal length, and one weight row.
+tile, K whose ranges are of unequal length or whose ends cut off weight groups
+of 2 and 4 pairs, and one weight row.
 
 Bars:
   plain     : against the float64 product of the fp16-rounded activations,
@@ -21,14 +22,24 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SHAPES = [  # (m, k, n), ranges on 256 CUs
-    (17, 3072, 48), (32, 3072, 3071), (33, 3072, 97), (64, 3456, 1000), (65, 15360, 193), (256, 3072, 3072),  # 8
-    (31, 1920, 18433), (129, 2688, 9000), (512, 1536, 3072),                                                # 4
-    (63, 768, 577), (200, 1152, 640), (1024, 1536, 3072),                                                   # 2
-    (19, 384, 1), (63, 384, 1500), (300, 3072, 9216), (130, 768, 30000), (1000, 1152, 9217),                # 1
-    # weight groups of 2 and 4 pairs cut off by a range's end, every tile
-    (33, 3456, 300), (500, 2688, 3071), (777, 1920, 3000), (1024, 8064, 3072), (400, 384, 9217), (1100, 1152, 9000),
-]
+# (m, k, n), by K ranges on 256 CUs
+RANGES = {
+    8: [(17, 3072, 48), (32, 3072, 3071), (33, 3072, 97), (64, 3456, 1000), (65, 15360, 193), (256, 3072, 3072),
+        (33, 3456, 300)],
+    4: [(31, 1920, 18433), (129, 2688, 9000), (512, 1536, 3072), (500, 2688, 3071)],
+    2: [(63, 768, 577), (200, 1152, 640), (1024, 1536, 3072), (300, 3072, 9216), (777, 1920, 3000),
+        (1024, 8064, 3072)],
+    1: [(19, 384, 1), (63, 384, 1500), (130, 768, 30000), (1000, 1152, 9217), (400, 384, 9217), (1100, 1152, 9000)],
+}
+SHAPES = [s for r in RANGES.values() for s in r]
+# (m, k, n, epilogue, split, kernel on 256 CUs): every tile, plain and packed
+PLANS = [(17, 3072, 48, "plain", 0, "k8 32x48"), (256, 3072, 3072, "plain", 0, "k8 64x48"),
+         (129, 2688, 9000, "plain", 0, "k4 32x96"), (512, 1536, 3072, "plain", 0, "k4 64x96"),
+         (200, 1152, 640, "plain", 0, "k2 64x96"), (63, 384, 1500, "plain", 0, "k1 32x192"),
+         (130, 768, 30000, "plain", 0, "k1 64x192"), (1000, 1152, 9217, "plain", 0, "k1 128x192"),
+         (64, 3456, 960, "packed_swiglu", 0, "k8 32x64"), (256, 3072, 3072, "packed_swiglu", 0, "k8 64x64"),
+         (512, 1536, 3072, "packed_swiglu", 0, "k4 64x128"), (200, 1152, 640, "packed_swiglu", 0, "k2 64x128"),
+         (1024, 1536, 3072, "packed_swiglu", 0, "k2 64x192"), (63, 384, 1472, "packed_swiglu", 0, "k1 32x192")]
 
 
 def say(msg):

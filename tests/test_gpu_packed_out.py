@@ -2,7 +2,7 @@
 activations (bonsai_b1_linear_packed_f16_to_packed).
 
 Bar (bit for bit): the fp32 columns equal the plain GEMM's output (the same
-tile kernel, the same K order), and the packed columns equal the packing
+K order, whichever kernel each runs), and the packed columns equal the packing
 the separate producers write from that output -- bonsai_b1_pack_act_f16_ld,
 bonsai_b1_gelu_tanh_pack_f16_ld or bonsai_b1_swiglu_pack_f16_ld -- which
 the producer tests pin against the oracle's layout.  Bytes outside the
@@ -59,12 +59,8 @@ CASES = [
     (256, 768, 2048, 192, "swiglu", 64, 1216),       # SwiGLU split inside a tile, into a column range
     (600, 3072, 21504, 9216, "gelu_tanh", 3072, 15360),  # C5 linear1 -> linear2's input
     (600, 3072, 27648, 9216, "swiglu", 3072, 12288),     # reference single block linear1 -> to_out's input
-    # 16x16 tile kernels (GELU and none; the plain reference runs the same
-    # kernel): 144 x 384 and 128 x 384 tiles, every column packed; split
-    # inside a wave (a block's halves in two waves: 2-byte half stores);
-    # a wave with one fp32 tile and one packed block (fewer stores than a
-    # full tile's: the next tile waits for everything); several tiles a
-    # work-group
+    # K-range tiles: every column packed, split points inside a wave's
+    # columns, column ranges, several tiles a work-group
     (288, 384, 768, 0, "gelu_tanh", 0, None),
     (288, 384, 768, 416, "gelu_tanh", 0, None),
     (288, 384, 768, 448, "none", 32, 400),
@@ -75,17 +71,46 @@ CASES = [
     # no activation, tiles wholly past the split point (the owner layout)
     (512, 384, 768, 0, "none", 0, None),
     (288, 384, 1152, 384, "none", 0, None),
-    # SwiGLU on 16x16 tiles (split on a 384-column tile boundary): every
-    # wave's 24 gates paired with their values, written as fp16 halves
+    # SwiGLU, from the first column and from a multiple of 384
     (512, 384, 768, 0, "swiglu", 0, None),
     (288, 384, 1152, 384, "swiglu", 0, None),
     (512, 384, 1536, 768, "swiglu", 32, 432),
     (4608, 384, 18432, 9216, "swiglu", 0, None),
-    # packed rows of 2^22 + 32 fp16 elements, past the range of a buffer
-    # resource over a tile's rows: the element-by-element stores
+    # packed rows of 2^22 + 32 fp16 elements
     (288, 384, 768, 0, "gelu_tanh", 0, 2**22 + 32),
     (512, 384, 1536, 0, "swiglu", 0, 2**22 + 32),
 ]
+
+# 16x16 tile kernels, 144 x 384 and 128 x 384 (m, k, n, split, act, column
+# offset, ldp, kernel on 256 CUs)
+CASES16 = [
+    # every column packed; split inside a wave (a block's halves in two waves:
+    # 2-byte half stores); a wave with one fp32 tile and one packed block
+    # (fewer stores than a full tile's: the next tile waits for everything)
+    (288, 384, 19968, 0, "gelu_tanh", 0, None, "144x384"),
+    (288, 384, 19968, 9632, "gelu_tanh", 0, None, "144x384"),
+    (288, 384, 19968, 9664, "none", 32, 10344, "144x384"),
+    (640, 384, 4992, 0, "gelu_tanh", 0, None, "128x384"),
+    (640, 384, 4992, 160, "gelu_tanh", 96, 4936, "128x384"),
+    # no activation, tiles wholly past the split point (the owner layout)
+    (288, 384, 19968, 9600, "none", 0, None, "144x384"),
+    (640, 384, 4992, 0, "none", 0, None, "128x384"),
+    # SwiGLU (split on a 384-column tile boundary): every wave's 24 gates
+    # paired with their values, written as fp16 halves
+    (288, 384, 19968, 9600, "swiglu", 0, None, "144x384"),
+    (384, 384, 4224, 0, "swiglu", 0, None, "128x384"),
+    (384, 384, 4224, 1536, "swiglu", 32, 1376, "128x384"),
+    # several tiles a work-group
+    (2736, 384, 18432, 4608, "gelu_tanh", 0, None, "144x384"),
+    (2736, 384, 18432, 9216, "swiglu", 0, None, "144x384"),
+    # packed rows of 2^22 + 32 fp16 elements, past the range of a buffer
+    # resource over a tile's rows: the element-by-element stores
+    (144, 384, 19968, 0, "gelu_tanh", 0, 2**22 + 32, "144x384"),
+    (128, 384, 12672, 0, "swiglu", 0, 2**22 + 32, "128x384"),
+]
+_EPILOGUE = {"none": "packed", "gelu_tanh": "packed_gelu", "swiglu": "packed_swiglu"}
+# (m, k, n, epilogue, split, kernel on 256 CUs)
+PLANS = [(c[0], c[1], c[2], _EPILOGUE[c[4]], c[3], c[7]) for c in CASES16]
 
 
 def _sweep(count=10, seed=2024):
@@ -111,7 +136,7 @@ def _sweep(count=10, seed=2024):
     return cases
 
 
-@pytest.mark.parametrize("m,k,n,split,act,col0,ldp", CASES + _sweep())
+@pytest.mark.parametrize("m,k,n,split,act,col0,ldp", CASES + [c[:7] for c in CASES16] + _sweep())
 def test_packed_output_equals_linear_then_producer(torch, b1, m, k, n, split, act, col0, ldp):
     from bonsai_b1 import synth
     say(f"packed-output linear m={m} k={k} n={n} split={split} act={act} col0={col0} ldp={ldp}")

@@ -394,20 +394,31 @@ def test_callback_deferred_checking(torch, b1):
     W.free()
 
 
+TAIL_KINDS = {"plain": "plain", "scaled": "plain", "gate_residual": "gate_residual", "swiglu": "swiglu",
+              "gelu_packed": "packed_gelu", "swiglu_packed": "packed_swiglu"}
+# (m, k, n, epilogue, split, kernel on 256 CUs) of the tests that are about one kernel
+PLANS = [(m, k, n, "plain", 0, p) for m, k, n, p in
+         [(256, 3072, 3072, "k8 64x48"), (512, 9216, 3072, "k4 64x96"), (512, 3072, 9216, "k1 32x192"),
+          (37, 15360, 384, "k8 32x48"), (200, 768, 600, "k2 64x96")]] + \
+        [(4240, 3072, 9216, e, 0, "128x512+64") for e in TAIL_KINDS.values()] + \
+        [(4592, 3072, 12288, "packed_swiglu", 0, "128x512+64"), (454, 384, 18560, "plain", 0, "128x512")]
+
+
 @pytest.mark.parametrize("m,n,ms,kind", [(4592, 12288, 4096, kd) for kd in
-                                          ("plain", "scaled", "gate_residual", "swiglu", "gelu_packed")] +
-                         [(4000, 9216, 3584, kd) for kd in ("plain", "gate_residual", "gelu_packed")])
+                                          ("plain", "scaled", "gate_residual", "swiglu", "gelu_packed",
+                                           "swiglu_packed")] +
+                         [(4000, 9216, 3584, kd) for kd in ("plain", "gate_residual", "gelu_packed")] +
+                         [(4240, 9216, 3584, kd) for kd in TAIL_KINDS])
 def test_tail_rows_as_half_height_tiles(torch, b1, m, n, ms, kind):
-    """M=4592 K=3072 N=12288 on 256 CUs runs its 768 full-round tiles of 128
-    rows, then rows 4096..4591 as 64-row tiles in a second launch (M=4000
-    N=9216: 504 tiles of rows [0, 3584) in two rounds, then the rest as
-    64-row tiles).  Every output is the same sum in the same order as in two
-    separate calls over rows [0, ms) and [ms, M), which take no such split:
-    bit for bit, for each epilogue kind.  (The plain reference goes through the
-    epilogue entry with no epilogue: the plain entry would split the
-    ~500-row call along K.)  With range-safe row scales, the scaled rows
-    equal the unscaled ones times their scales.  (M is a multiple of
-    neither 128 nor 144, so no 16x16 tile kernel takes the plain forms.)"""
+    """M=4240 K=3072 N=9216 on 256 CUs runs 504 tiles of 128 x 512, rows [0,
+    3584), in two rounds, then rows 3584..4239 as 64-row tiles in a second
+    launch, with every epilogue (M=4592 N=12288 with a packed SwiGLU output
+    too: 768 tiles of rows [0, 4096), then the rest; their other epilogues and
+    M=4000 run K-range tiles).  Every output is the same sum in the same order
+    as in two separate calls over rows [0, ms) and [ms, M), which take other
+    kernels: bit for bit, for each epilogue kind.  With range-safe row scales,
+    the scaled rows equal the unscaled ones times their scales.  (M is a
+    multiple of neither 128 nor 144, so no 16x16 tile kernel takes them.)"""
     from bonsai_b1 import synth
     k = 3072
     say(f"tail rows as half-height tiles: ({m},{k},{n}) {kind} "
@@ -432,15 +443,15 @@ def test_tail_rows_as_half_height_tiles(torch, b1, m, n, ms, kind):
             return b1.linear_packed_f16_epi(p, w, k, n, rows, "gate_residual", gate=gate, residual=res[r0:r0 + rows])
         if kind == "swiglu":
             return b1.linear_packed_f16_epi(p, w, k, n, rows, "swiglu")
-        _, po = b1.linear_packed_f16_to_packed(p, w, k, n, rows, 0, "gelu_tanh")
+        _, po = b1.linear_packed_f16_to_packed(p, w, k, n, rows, 0,
+                                               "gelu_tanh" if kind == "gelu_packed" else "swiglu")
         return po
 
     g = torch.Generator(device="cuda").manual_seed(63)
     gate = 0.1 * torch.randn(n, device="cuda", generator=g)
     res = torch.randn((m, n), device="cuda", generator=g)
     if kind == "scaled":
-        # the scaled entry splits a 512-row call along K too; its rows are the
-        # unscaled products times their scales, one fp32 multiply each
+        # rows are the unscaled products times their scales, one fp32 multiply each
         full = b1.linear_packed_f16_scaled(pa, rsc, w, k, n, m)
         ref = b1.linear_packed_f16_epi(pa, w, k, n, m, "none") * rsc[:, None]
         torch.cuda.synchronize()
@@ -511,17 +522,22 @@ def pack_area_bytes(m, k):
     return (m * k * 2 + 255) // 256 * 256 + (m * 4 + 255) // 256 * 256
 
 
-def unsplit_linear(torch, b1, a, w, n, mode):
-    """The fp32 entry with a workspace that holds the packing only, so the
-    GEMM runs unsplit along K."""
+def own_workspace_linear(torch, b1, a, w, n, mode):
+    """The fp32 entry with the caller's workspace, of the packing's size."""
     ws = torch.empty(pack_area_bytes(*a.shape), dtype=torch.uint8, device="cuda")
     return b1.linear(a, w, n, mode=mode, workspace=ws)
+
+
+def one_range_linear(torch, b1, a, w, n):
+    """The GEMM that converts the activations itself (a workspace too small
+    for the packing), which sums K as one range."""
+    return b1.linear(a, w, n, mode="gemm", workspace=torch.empty(16, dtype=torch.uint8, device="cuda"))
 
 
 @pytest.mark.parametrize("m,k,n", [(200, 768, 600), (128, 384, 512), (1, 384, 40)])
 def test_linear_packed_matches_fused_entry(torch, b1, m, k, n):
     """pack + linear_packed gives bit-for-bit what bonsai_b1_linear_f32 gives
-    in GEMM mode (same kernels, split along K the same way), including a
+    in GEMM mode (same kernels, the same K ranges), including a
     padded output stride."""
     from bonsai_b1 import synth
     a = synth.device_activations(m, k, 41)
@@ -968,9 +984,9 @@ def test_linear_batch_group_order_and_range(torch, b1):
     assert bool(torch.isfinite(ga[[0, 1, 3, 11]]).all())
 
 
-# ---------------------------------------------------------------- split-K --
+# --------------------------------------------------------------- K ranges --
 
-SPLIT_CASES = [  # (m, k, n): shapes whose 128 x 512 tiles leave most CUs idle
+SPLIT_CASES = [  # (m, k, n): shapes with few output tiles, whose K is summed in ranges
     (256, 3072, 3072),    # C1: 12 tiles
     (512, 9216, 3072),    # Klein text stream FF-out: 24 tiles, long K
     (512, 3072, 9216),    # Klein text stream q/k/v
@@ -981,38 +997,39 @@ SPLIT_CASES = [  # (m, k, n): shapes whose 128 x 512 tiles leave most CUs idle
 
 
 @pytest.mark.parametrize("m,k,n", SPLIT_CASES)
-def test_split_k(torch, b1, m, k, n):
-    """GEMMs split along K (work units of a tile and a K range, fp32 partial
-    products summed in a fixed order by a second kernel): against the same
-    GEMM unsplit, the difference is the summation order alone (<= 1e-5 of
-    the output rms); against EXACT, the FAST bar; two runs are bit for bit
-    the same; a padded, non-multiple-of-4 output stride is written only in
-    its columns."""
+def test_split_k(torch, b1, gemm_plan, m, k, n):
+    """GEMMs whose K is summed in ranges (a work-group's waves take a range
+    each, the partial tiles are added in LDS in range order): against the
+    converting GEMM, which sums one range, the difference is the summation
+    order alone (<= 1e-5 of the output rms); against EXACT, the FAST bar; two
+    runs are bit for bit the same; a padded, non-multiple-of-4 output stride is
+    written only in its columns."""
     from bonsai_b1 import synth
-    say(f"split-K ({m},{k},{n})")
+    say(f"K ranges ({m},{k},{n})")
     a = synth.device_activations(m, k, 45)
     w = synth.device_packed_weights(n, k, 46)
     y = b1.linear(a, w, n, mode="gemm")
     y2 = b1.linear(a, w, n, mode="gemm")
-    yu = unsplit_linear(torch, b1, a, w, n, "gemm")
+    yu = one_range_linear(torch, b1, a, w, n)
     ye = b1.linear(a, w, n, mode="exact")
     out = torch.full((m, n + 3), 7.0, device="cuda")
     b1.linear(a, w, n, out=out[:, :n], mode="gemm")
     torch.cuda.synchronize()
-    assert torch.equal(y, y2), "split-K is deterministic"
+    assert torch.equal(y, y2), "the ranges are added in order"
     rms = float(yu.pow(2).mean().sqrt())
     d = float((y - yu).abs().max())
-    say(f"  split vs unsplit max |diff| {d:.3e} (rms {rms:.3e}); identical: {bool(torch.equal(y, yu))}")
+    say(f"  ranges vs one range max |diff| {d:.3e} (rms {rms:.3e}); identical: {bool(torch.equal(y, yu))}")
     assert d <= 1e-5 * rms
-    assert_fast_close(y.cpu().numpy(), ye.cpu().numpy(), f"split-K {(m, k, n)} vs exact")
+    assert torch.equal(y, yu) == gemm_plan(m, k, n).startswith("k1 "), "more than one range"
+    assert_fast_close(y.cpu().numpy(), ye.cpu().numpy(), f"K ranges {(m, k, n)} vs exact")
     assert torch.equal(out[:, :n], y)
     assert bool((out[:, n:] == 7.0).all()), "columns past out_dim untouched"
 
 
 def test_split_k_counts_nonfinite(torch, b1):
-    """The non-finite count comes from the summed outputs (the partials are
-    not counted): an infinite activation makes its row's outputs non-finite
-    in the split GEMM as in the unsplit one."""
+    """The non-finite count comes from the summed outputs (the partial tiles
+    are not counted): an infinite activation makes its row's outputs
+    non-finite in the GEMM over K ranges as in the converting one."""
     from bonsai_b1 import synth
     m, k, n = 256, 3072, 3072
     a = synth.device_activations(m, k, 47)
@@ -1021,19 +1038,19 @@ def test_split_k_counts_nonfinite(torch, b1):
     nf = torch.zeros(1, dtype=torch.int32, device="cuda")
     y = b1.linear(a, w, n, mode="gemm", nonfinite=nf)
     nfu = torch.zeros(1, dtype=torch.int32, device="cuda")
-    ws = torch.empty(pack_area_bytes(m, k), dtype=torch.uint8, device="cuda")
-    yu = b1.linear(a, w, n, mode="gemm", nonfinite=nfu, workspace=ws)
+    yu = b1.linear(a, w, n, mode="gemm", nonfinite=nfu,
+                   workspace=torch.empty(16, dtype=torch.uint8, device="cuda"))
     torch.cuda.synchronize()
     bad = int((~torch.isfinite(y)).sum())
-    say(f"  non-finite outputs {bad}, counted {int(nf.item())} split / {int(nfu.item())} unsplit")
+    say(f"  non-finite outputs {bad}, counted {int(nf.item())} in ranges / {int(nfu.item())} in one")
     assert bad == n and int(nf.item()) == bad and int(nfu.item()) == int((~torch.isfinite(yu)).sum())
 
 
 @pytest.mark.parametrize("m,k,n,splits", [(256, 3072, 3072, 8), (200, 768, 600, 2)])
 def test_split_k_equals_per_range_composition(torch, b1, m, k, n, splits):
-    """Bit for bit, on every one of several launches: the split GEMM equals
-    the sum, in range order, of unsplit GEMMs over the K ranges (sliced
-    activations and weights).  Regression test for an epilogue that
+    """Bit for bit, on every one of several launches: the GEMM over `splits`
+    K ranges equals the sum, in range order, of GEMMs over each (sliced
+    activations and weights, 384 of K: one range).  Regression test for an epilogue that
     rearranged accumulators across lanes before storing and intermittently
     stored stale values of one accumulator register in four lanes."""
     from bonsai_b1 import synth
@@ -1044,7 +1061,7 @@ def test_split_k_equals_per_range_composition(torch, b1, m, k, n, splits):
     ref = None
     for s in range(splits):
         ws_ = wr[:, s * kr // 32:(s + 1) * kr // 32, :].contiguous().view(-1)
-        part = unsplit_linear(torch, b1, a[:, s * kr:(s + 1) * kr].contiguous(), ws_, n, "gemm")
+        part = own_workspace_linear(torch, b1, a[:, s * kr:(s + 1) * kr].contiguous(), ws_, n, "gemm")
         ref = part if ref is None else ref + part
     for run in range(6):
         y = b1.linear(a, w, n, mode="gemm")
@@ -1054,18 +1071,19 @@ def test_split_k_equals_per_range_composition(torch, b1, m, k, n, splits):
         assert nbad == 0
 
 
-@pytest.mark.parametrize("m,k,n", [(200, 384, 600), (256, 768, 1024)])
+@pytest.mark.parametrize("m,k,n", [(200, 384, 600), (256, 768, 1024), (454, 384, 18560)])
 def test_one_tile_per_work_group_repeats(torch, b1, m, k, n):
-    """Unsplit GEMMs with one output tile per work-group (the epilogue right
-    after the last MFMAs, nothing in between): every launch gives the same
-    bits and stays within the FAST bar of EXACT."""
+    """GEMMs with one output tile per work-group (the epilogue right after the
+    last MFMAs, nothing in between), of K-range tiles and (454 x 384 -> 18560)
+    of the 128 x 512 kernel: every launch gives the same bits and stays within
+    the FAST bar of EXACT."""
     from bonsai_b1 import synth
     a = synth.device_activations(m, k, 49)
     w = synth.device_packed_weights(n, k, 50)
     ye = b1.linear(a, w, n, mode="exact")
-    first = unsplit_linear(torch, b1, a, w, n, "gemm")
+    first = own_workspace_linear(torch, b1, a, w, n, "gemm")
     for run in range(8):
-        y = unsplit_linear(torch, b1, a, w, n, "gemm")
+        y = own_workspace_linear(torch, b1, a, w, n, "gemm")
         torch.cuda.synchronize()
         assert torch.equal(y, first), f"launch {run}"
     assert_fast_close(first.cpu().numpy(), ye.cpu().numpy(), f"one tile per WG {(m, k, n)}")

@@ -57,25 +57,29 @@ def test_strided_producers_build_concatenated_input(torch, b1, m, k1, k2):
         w = synth.device_packed_weights(384, k, 73)
         y = b1.linear_packed_f16(buf, w, k, 384, m)
         cat = torch.cat([a1, b1.gelu_tanh(a2.contiguous())], 1)
-        # the fp32 entry, split along K as the packed entry splits
+        # the fp32 entry, the same K ranges as the packed entry
         yr = b1.linear(cat, w, 384)
         torch.cuda.synchronize()
         assert torch.equal(y, yr)
 
 
-# (4600: the 128 x 512 kernel; 4608 and the Klein FF-in's 4096: the 16x16
+# (4480: the 128 x 512 kernel; 4608 and the Klein FF-in's 4096: the 16x16
 # tile kernels, 144 x 384 and 128 x 384, the fused SwiGLU pairing each
-# wave's 24 gates with their values)
+# wave's 24 gates with their values; the others: K-range tiles)
+# (m, k, n, epilogue, split, kernel on 256 CUs)
+PLANS = [(4480, 3072, 18432, "swiglu", 0, "128x512"), (4608, 3072, 18432, "swiglu", 0, "144x384"),
+         (4096, 3072, 18432, "swiglu", 0, "128x384"), (4600, 3072, 18432, "swiglu", 0, "k1 128x192")]
+
+
 @pytest.mark.parametrize("m,k,h", [(300, 1152, 768), (64, 384, 96), (4600, 3072, 9216), (4608, 3072, 9216),
-                                   (4096, 3072, 9216)])
+                                   (4096, 3072, 9216), (4480, 3072, 9216)])
 def test_swiglu_pack_matches_fused_epilogue(torch, b1, oracle, m, k, h):
     from bonsai_b1 import synth
     say(f"swiglu pack m={m} k={k} h={h}")
     a = synth.device_activations(m, k, 74)
     w = synth.device_packed_weights(2 * h, k, 75)
     pa = b1.pack_act_f16(a)
-    # [gates | values], unsplit along K as the fused epilogue runs (a
-    # workspace too small for split-K partials)
+    # [gates | values], the K ranges of the fused epilogue
     y = b1.linear_packed_f16(pa, w, k, 2 * h, m, workspace=torch.empty(16, dtype=torch.uint8, device="cuda"))
     p1 = b1.swiglu_pack_f16(y)
     out = b1.linear_packed_f16_epi(pa, w, k, 2 * h, m, "swiglu")  # fp32 [m, h]

@@ -9,14 +9,13 @@ Bars (those of tests/test_gpu_parity.py and tests/test_gpu_epilogue.py):
                   |y - ref| / max(|ref|, rms(ref)) <= 1e-2, cosine >= 0.9999.
   gate-residual : bit for bit numpy's float32 residual + gate * y, y the
                   library's own linear in the same mode over a workspace
-                  that holds the packing only (the GEMM then runs unsplit
-                  along K, as the fused epilogue does).
+                  that holds the packing.
   Columns past out_dim keep their sentinel in every mode.
 The shapes are drawn so that every kernel choice of the library meets
 ragged edges: M from 1 to 1300 (the small-M kernels up to several rounds of
 tiles), K any multiple of 64 up to 4608 (K % 384 != 0 takes the
 fused-conversion GEMM, K % 256 != 0 the fallback small-M kernel), N from 1
-to 2600 (partial tiles, split-K and half-height tails where they apply),
+to 2600 (partial tiles and K ranges where they apply),
 and padded row strides.
 """
 import random
@@ -145,7 +144,7 @@ def _draw_swiglu(count, seed):
 @pytest.mark.parametrize("m,k,n,mode,lda", _draw_swiglu(16, 7))
 def test_random_shape_swiglu(torch, b1, m, k, n, mode, lda):
     """out[:, j] = silu(y[:, j]) * y[:, H + j] against that formula in
-    float64 on the library's own unsplit linear y, per element within
+    float64 on the library's own linear y, per element within
     1e-6 of the result; columns past H untouched."""
     from bonsai_b1 import synth
     say(f"random SwiGLU ({m},{k},{n}) {mode} lda={lda}")
@@ -378,8 +377,8 @@ def test_random_packed_entry(torch, b1, m, k, n):
     """bonsai_b1_linear_packed_f16 over pack_act_f16 of the activations gives
     the fp32 entry's outputs bit for bit: its FAST mode (M > 16 or K % 256
     == 0, the small-M kernel at M <= 16) or its GEMM mode (M <= 16 with K %
-    256 != 0, where the packed entry keeps the GEMM tile), split along K
-    alike."""
+    256 != 0, where the packed entry keeps the GEMM), in the same K
+    ranges."""
     from bonsai_b1 import synth
     mode = "auto" if (m > 16 or k % 256 == 0) else "gemm"
     say(f"random packed entry ({m},{k},{n}) vs fp32 {mode}")

@@ -5,7 +5,7 @@ The reference sums any finite fp32 activation in fp32
 (src/b1_0_kernel.h:117-134,218-228).  FAST mode rounds activations to fp16,
 whose largest finite value is 65504; the fp32 entry points therefore pack a
 row whose largest |a| would overflow (>= 65520) times 2^-e and multiply its
-outputs by 2^e (the packed GEMM, split-K, grouped small-M ops of a batch,
+outputs by 2^e (the packed GEMM, its K ranges, grouped small-M ops of a batch,
 the fused epilogues), and, where a kernel converts activations itself (the
 small-M kernel, GEMMs without a workspace), compute such rows again in
 EXACT arithmetic.
@@ -82,8 +82,8 @@ def assert_rows_close(y, ref, what):
 # (m, k, n, mode, workspace): "lib" = the library's own, None = a too-small
 # caller workspace (the kernels that convert activations themselves)
 PATHS = [
-    (2048, 768, 4608, "auto", "lib"),     # packed GEMM, unsplit (192 tiles of 128 x 384)
-    (256, 3072, 3072, "auto", "lib"),     # packed GEMM split along K (C1)
+    (2048, 768, 4608, "auto", "lib"),     # packed GEMM, one K range (192 tiles of 128 x 384)
+    (256, 3072, 3072, "auto", "lib"),     # packed GEMM in 8 K ranges (C1)
     (8, 3072, 4096, "auto", "lib"),       # small-M kernel: exact rows inside it
     (16, 768, 640, "gemm", "lib"),        # GEMM tile for a few rows
     (300, 768, 600, "gemm", None),        # fused-conversion GEMM + exact rows
@@ -278,9 +278,9 @@ def test_packed_small_m_group_under_capture_without_workspace(torch, b1):
 
 @pytest.mark.parametrize("m,k,n", [(256, 3072, 3072), (512, 9216, 3072), (37, 15360, 384)])
 def test_packed_entry_splits_like_fp32_entry(torch, b1, m, k, n):
-    """bonsai_b1_linear_packed_f16 splits along K exactly as
-    bonsai_b1_linear_f32 does for the same shape (the library's workspace
-    or the caller's), so the two entries agree bit for bit."""
+    """bonsai_b1_linear_packed_f16 sums the K ranges that
+    bonsai_b1_linear_f32 sums for the same shape, with or without a workspace
+    of the size its query reports, so the two entries agree bit for bit."""
     from bonsai_b1 import synth
     say(f"packed entry split ({m},{k},{n})")
     a = synth.device_activations(m, k, 91)
@@ -289,7 +289,7 @@ def test_packed_entry_splits_like_fp32_entry(torch, b1, m, k, n):
     packed = b1.pack_act_f16(a)
     y = b1.linear_packed_f16(packed, w, k, n, m)
     need = b1.linear_packed_workspace_bytes(m, k, n)
-    assert need > 0, "this shape splits along K"
+    assert need > 0, "the size that K ranges split over work-groups took"
     ws = torch.empty(need, dtype=torch.uint8, device="cuda")
     y2 = b1.linear_packed_f16(packed, w, k, n, m, workspace=ws)
     torch.cuda.synchronize()
@@ -300,8 +300,8 @@ def test_packed_entry_splits_like_fp32_entry(torch, b1, m, k, n):
 @pytest.mark.parametrize("m,k,n", [(256, 3072, 3072), (2048, 768, 4608), (8, 3072, 4096)])
 def test_scaled_halves_equal_fp32_entry(torch, b1, m, k, n):
     """bonsai_b1_pack_act_f16_scaled + bonsai_b1_linear_packed_f16_scaled
-    give bonsai_b1_linear_f32's FAST results bit for bit (split-K and
-    unsplit GEMMs), on activations beyond the fp16 range too; small-M
+    give bonsai_b1_linear_f32's FAST results bit for bit (GEMMs of
+    one and of several K ranges), on activations beyond the fp16 range too; small-M
     batches agree on rows within range (the fp32 entry computes the others
     in EXACT arithmetic: both within the FAST bar of the oracle).  On rows
     within range the scaled packing is bonsai_b1_pack_act_f16's, with

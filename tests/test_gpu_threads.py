@@ -8,7 +8,7 @@ waits for the kernels already queued on it).  Ten host threads, each on a
 stream of its own, run linears whose workspace needs grow call by call, so
 buffers are replaced and evicted while other threads' calls are in flight.
 Bar: every output equals the same call made alone on one stream
-beforehand, bit for bit (same kernels, same split along K).
+beforehand, bit for bit (same kernels, same K ranges).
 The per-thread non-finite counter of the deferred callback is checked the
 same way: each thread's count is its own.  The callback queues on
 hipStreamPerThread, one handle value that names each thread's own stream:
@@ -166,8 +166,7 @@ def test_per_thread_default_stream(torch, b1):
     """hipStreamPerThread, one handle value naming a different stream in
     each thread, passed to the fp32 entry by ten threads at once, four calls
     each with no synchronisation between them (each call packs its input
-    into the library's workspace and splits the GEMM along K into partials
-    there): every output bit for bit the same call made alone.  The library
+    into the library's workspace): every output bit for bit the same call made alone.  The library
     keeps such a stream's workspace per calling thread; shared by handle
     value, one thread's packing would be read by another's GEMM."""
     from bonsai_b1 import capi, synth

@@ -2,12 +2,13 @@
 
 The packed GEMM runs one of them for full-tile shapes whose 128 x 512 tiles
 would quantise worse on the CUs (M % 144 or M % 128 == 0, N % 384 == 0,
-K % 384 == 0, no split along K, fewer rounds counted in 128 x 512 tiles:
-on 256 CUs e.g. 288 x 384 -> 768, 1440 x 1152 -> 3072 and the Flux shapes
-M = 4608 with N = 3072, 9216, 12288 or 21504 take 144 x 384 tiles; 512 x
-384 -> 768, 2048 x 768 -> 4608 and the Klein image shapes M = 4096 with
-N = 3072, 9216 or 18432 take 128 x 384 tiles).  Checked here on such
-shapes, through the fp32, packed and epilogue entries:
+K % 384 == 0, one K range, fewer rounds counted in 128 x 512 tiles) and whose
+K-range tiles model no faster: on 256 CUs e.g. 288 x 384 -> 19968, 2736 x 768
+-> 18432 and the Flux shapes M = 4608 with N = 3072, 9216, 12288 or 21504 take
+144 x 384 tiles; 640 x 384 -> 4992, 2048 x 768 -> 4608 and the Klein image
+shapes M = 4096 with N = 3072, 9216 or 18432 take 128 x 384 tiles.  Checked
+here on such shapes, and on three smaller ones of full tiles that run K-range
+tiles, through the fp32, packed and epilogue entries:
 
   * the FAST bar against the float64 oracle (per element
     |y - ref| / max(|ref|, rms(ref)) <= 1e-2 and cosine >= 0.9999);
@@ -29,9 +30,14 @@ pytestmark = pytest.mark.gpu
 
 TOL_REL = 1e-2
 TOL_COS = 0.9999
-SHAPES144 = [(288, 384, 768), (1440, 1152, 3072), (4608, 3072, 3072)]
-SHAPES128 = [(512, 384, 768), (2048, 768, 4608), (4096, 3072, 9216)]
-SHAPES = SHAPES144 + SHAPES128
+SHAPES144 = [(288, 384, 19968), (2736, 768, 18432), (4608, 3072, 3072)]
+SHAPES128 = [(640, 384, 4992), (2048, 768, 4608), (4096, 3072, 9216)]
+KRANGE = [(288, 384, 768), (1440, 1152, 3072), (512, 384, 768)]
+SHAPES = SHAPES144 + SHAPES128 + KRANGE
+# (m, k, n, epilogue, split, kernel on 256 CUs)
+PLANS = [s + (e, 0, p) for e in ("plain", "gate_residual", "swiglu")
+         for p, shapes in (("144x384", SHAPES144), ("128x384", SHAPES128)) for s in shapes] + \
+        [(288, 384, 768, "plain", 0, "k1 32x192"), (1440, 1152, 3072, "plain", 0, "k1 64x192")]
 
 
 def say(msg):
@@ -103,7 +109,7 @@ def test_tiles16_against_oracle_and_entries(torch, b1, oracle, m, k, n):
     assert bool((big[:, n] == 7.0).all())
 
 
-@pytest.mark.parametrize("m,k,n", SHAPES144[:2] + SHAPES128[:2])
+@pytest.mark.parametrize("m,k,n", SHAPES144[:2] + SHAPES128[:2] + KRANGE)
 def test_tiles16_swiglu_scalar_store(torch, b1, m, k, n):
     """The fused SwiGLU epilogue into rows whose stride is not a multiple
     of 4 (element stores, the owner waves' block layout) gives the bits of
@@ -123,7 +129,7 @@ def test_tiles16_swiglu_scalar_store(torch, b1, m, k, n):
     assert bool((odd[:, h] == 7.0).all())
 
 
-@pytest.mark.parametrize("m,k,n", SHAPES144[:2] + SHAPES128[:2])
+@pytest.mark.parametrize("m,k,n", SHAPES144[:2] + SHAPES128[:2] + KRANGE)
 def test_tiles16_gate_residual(torch, b1, m, k, n):
     """out = residual + gate * y, fused, equals the fp32 multiply then add on
     the plain y; in place (residual = out) too."""
@@ -150,7 +156,7 @@ def test_tiles16_gate_residual(torch, b1, m, k, n):
     assert torch.equal(got2, want), "fp32 epilogue entry"
 
 
-@pytest.mark.parametrize("m,k,n", [(1440, 1152, 3072), (2048, 768, 4608)])
+@pytest.mark.parametrize("m,k,n", [(2736, 768, 18432), (2048, 768, 4608), (1440, 1152, 3072)])
 def test_tiles16_rows_beyond_fp16_and_nonfinite(torch, b1, oracle, m, k, n):
     from bonsai_b1 import synth
     a = synth.device_activations(m, k, 206)

@@ -1,7 +1,7 @@
 """bonsai_b1_linear_f32_noalloc: the entry point that allocates nothing.
 
 It runs the kernels of bonsai_b1_linear_f32 with their workspace (the fp16
-packing and the split-K partials) in a static device array, so its outputs
+packing) in a static device array, so its outputs
 must equal bonsai_b1_linear_f32's bit for bit.  Called through the C ABI
 with raw device pointers.  Two calls in a row, the second smaller, so the
 second runs over what the first left in the array; a call needing more
@@ -41,9 +41,9 @@ def _call(lib, torch, fn, a, w, n, out, mode):
                             capi.MODES[mode], None, stream)
 
 
-# (M, K, N, mode): the first needs the packing plus split-K partials
-# (256 x 3072 x 3072 splits K eight ways on 256 CUs: 1.5 MB + 25.2 MB), the
-# second a smaller packing over the first one's leftovers, then small-M
+# (M, K, N, mode): the first needs 1.5 MB of packing (256 x 3072 x 3072, eight
+# K ranges on 256 CUs), the second a smaller packing over the first one's
+# leftovers, then small-M
 # and EXACT calls that need none.
 SEQUENCE = [(256, 3072, 3072, "auto"), (160, 768, 600, "gemm"), (8, 3072, 4096, "auto"), (5, 256, 40, "exact")]
 
@@ -106,8 +106,7 @@ def test_noalloc_takes_unaligned_call_of_any_size(torch, lib):
 def test_noalloc_under_graph_capture(torch, lib):
     """Captured on a stream the library has never seen (so it owns no
     workspace for it, and a capture cannot allocate one), the no-alloc entry
-    still runs the packed GEMM, split along K (256 x 3072 x 3072: 26.7 MB of
-    packing and partials); every replay equals the eager result, with other
+    still runs the packed GEMM (256 x 3072 x 3072 in eight K ranges); every replay equals the eager result, with other
     no-alloc calls between the replays."""
     from bonsai_b1 import capi, synth
     m, k, n = 256, 3072, 3072
