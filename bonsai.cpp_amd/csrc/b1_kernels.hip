@@ -333,7 +333,7 @@ __device__ __forceinline__ void exact_rows(uint64_t (&row)[R], const uint16_t *w
 // bytes an activation, so wide tiles suit many tokens; with few, a tile's
 // serial K loop is what takes the time and small tiles fill the CUs
 // (launch_fused picks).  Every tile sums K in the same order: the same bits.
-// us with 128 x 512 tiles only -> now: M=1000 K=2048 N=5504 58.8 -> 40.2,
+// us with 128 x 512 tiles only -> now: M=1000 K=2048 N=5504 58.8 -> 40.8,
 // M=77 K=2048 N=5504 50 -> 21 (kernel alone).
 //
 // A row holding an |a| >= 65520 (or an inf), which fp16 cannot take, is not
@@ -3779,7 +3779,7 @@ double persistent_gemm_us(int M, int K, int N, int num_cus) {
 // 222 and 225, M=4096 N=12288 261 and 270).
 //  * Packed outputs, by packed_tile_us: 2 % better (SwiGLU: M=4592 K=3072
 //    N=12288 310 and 320, M=3744 K=768 N=19456 126 and 147, M=1024 K=3072
-//    N=18432 126 and 118).  Over 713 shapes of 300 to 4608 tokens K-range tiles
+//    N=18432 126 and 118).  Over 713 shapes of 224 to 4605 tokens K-range tiles
 //    are then taken where the persistent kernel is over 3 % faster 8 times, by
 //    up to 6 %; with the plain model and 7 %, 68 times, by up to 26 %.
 //  * Gate and residual over 512 MB of residual and output, twice the

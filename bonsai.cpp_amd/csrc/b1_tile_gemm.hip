@@ -33,10 +33,11 @@ using T1b = TileCfg<128, 48, 4, 1, 64, 2, 4>;
 
 // Time model of a launch, in microseconds, from launches of every tile over
 // 32 to 2048 tokens, K 1536 to 9216, N 3072 to 18432 on 256 CUs (most within
-// 10 %; up to 4608 tokens the 128-row tile takes up to 8 % more than modelled,
-// M=4592 N=12288 307 us for 285): a CU runs q tiles (rounded up), `occ` at a time; each adds e + c b
-// to a busy CU, b = K / 32 / KG blocks per range, and what is left at the end
-// takes e1 + c1 b at least, a tile's time alone.
+// 10 %; up to 4608 tokens the 128-row tile takes up to 13 % more than modelled,
+// M=4592 N=12288 307 us for 285, 23 % at K = 768): a CU runs q tiles (rounded
+// up), `occ` at a time; each adds e + c b to a busy CU, b = K / 32 / KG blocks
+// per range, and what is left at the end takes e1 + c1 b at least, a tile's
+// time alone.
 struct TileCost {
     int occ;
     double e, c, e1, c1;
